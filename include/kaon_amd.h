@@ -118,7 +118,7 @@ typedef struct KaonTensor {
   int64_t n;              /* R * C */
   /* workspace offsets, in 4-byte words from the workspace base (kaon_plan) */
   int64_t ws_row;         /* 5 arrays of R words: mu, rf, rs, amax, oldscale */
-  int64_t ws_col;         /* cf [C] */
+  int64_t ws_col;         /* cf [C + 8]: the column factors, the last 8 wrapped around */
   int64_t ws_part;        /* column partials [2][ngroups][C], one row per run: of q = g^2 (+eps1)
                              and, for the RMS clip, of g^2 / row */
   int64_t ws_blk;         /* 4-bit: 2 arrays of nblocks words: amax, oldscale */

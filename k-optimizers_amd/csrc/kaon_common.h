@@ -41,6 +41,13 @@ struct Ws {
   }
 };
 
+// A column factor and its wrapped copies: cf holds C + 8 words, cf[j + k C] for
+// every j + k C < C + 8, so that eight consecutive reads from any column run on
+// into the next row's columns (the flat chunks of kaon_flat.hip).
+__device__ __forceinline__ void put_cf(KAON_G float* cf, int64_t C, int64_t j, float v) {
+  for (int64_t q = j; q < C + 8; q += C) cf[q] = v;
+}
+
 // Streaming accesses: the gradient, parameter and momentum streams of a
 // 2.6B-param step are far larger than the caches, so they are loaded and
 // stored as non-temporal accesses (NT); small reused arrays (column
@@ -119,11 +126,13 @@ __device__ __forceinline__ int chunk_cnt(int64_t c, int64_t C) {
   return j0 >= C ? 0 : (int)min<int64_t>(8, C - j0);
 }
 
-// Zero what phase 5 accumulates with atomics (keep-count; 4-bit block absmax
-// of blocks that straddle rows).  Run by the phase-1 slice.
+// Zero what phase 5 accumulates with atomics (keep-count; int8 row absmax, 4-bit
+// block absmax).  Run by the phase-1 slice.
 __device__ void zero_accumulators(const KaonTensor& T, const KaonItem& it, const Ws& ws, int codec) {
   if (it.row0 == 0 && threadIdx.x == 0) ((KAON_G uint32_t*)ws.scal(T))[1] = 0u;
-  if (codec == KAON_MOM_4BIT) {
+  if (codec == KAON_MOM_INT8) {
+    for (int64_t r = it.row0 + threadIdx.x; r < (int64_t)it.row0 + it.nrows; r += KAON_WG) ws.ramax(T)[r] = 0u;
+  } else if (codec == KAON_MOM_4BIT) {
     const int64_t e_begin = (int64_t)it.row0 * T.C;
     const int64_t e_end = (int64_t)(it.row0 + it.nrows) * T.C;
     if (e_end <= e_begin) return;
@@ -252,6 +261,17 @@ int torch_clip(const KaonLaunch& L, Ws ws, const KaonHyper& h, int32_t t0, int32
 
 // A phase-5/6 kernel over work items: (descriptors, items, workspace, hyper-parameters).
 using ElemFn = void (*)(const KaonTensor*, const KaonItem*, Ws, KaonHyper);
+
+// The general phase-5/6 kernels, by flat chunks, for the launch's types and
+// codec (kaon_flat.hip); nullptr for a combination the optimizer does not step.
+ElemFn flat_ada5(const KaonHyper& h, int codec);
+ElemFn flat_ada6(const KaonHyper& h, int codec);
+ElemFn flat_lion5(const KaonHyper& h, int codec);
+ElemFn flat_lion6(const KaonHyper& h, int codec);
+ElemFn flat_muon5(const KaonHyper& h, int codec);
+ElemFn flat_muon6(const KaonHyper& h, int codec);
+ElemFn flat_pnm5(const KaonHyper& h, int codec);
+ElemFn flat_pnm6(const KaonHyper& h, int codec);
 
 // The specialized phase-5/6 kernel for (optimizer, phase 5 or 6, codec, FF_*
 // flags), or nullptr when none is compiled for that configuration

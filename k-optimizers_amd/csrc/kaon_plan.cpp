@@ -266,7 +266,7 @@ extern "C" int kaon_plan(const KaonPlanArgs* args, KaonTensor* descs, int32_t n,
       t.ws_part = off;
       off = round4(off + t.n / t.fb_c);
     } else if (t.factored && !t.full_v) {
-      off = round4(off + t.C);
+      off = round4(off + t.C + 8);  // the column factors and their wrapped copies
       t.ws_part = off;
       // the column partials of G^2 and, after them, of the clip's G^2 / row
       off = round4(off + 2 * (int64_t)t.ngroups * t.C);

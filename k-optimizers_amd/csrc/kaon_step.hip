@@ -546,7 +546,7 @@ __global__ __launch_bounds__(KAON_WG) void k_fin(const KaonTensor* __restrict__ 
       const float cs = run_sum(part, T.ngroups, C, j);
       const float nc = klerp(T.col[j], cs / (float)R, hp.w2);
       T.col[j] = nc;
-      cf[j] = 1.0f / sqrtf(nc);
+      put_cf(cf, C, j, 1.0f / sqrtf(nc));
       if (alg) a = a + run_sum(part2, T.ngroups, C, j) / nc;
     }
     if (alg) {
@@ -1221,465 +1221,6 @@ __global__ __launch_bounds__(KAON_WG) void k_muon_norm(const KaonTensor* __restr
   if (lane == 0) ws.scal(T)[2] = rbf(rbf(sqrtf(ss)) + 1e-7f);
 }
 
-// Per-chunk body of phases 5 and 6.  Row context (mu, rf, scales) is uniform
-// over the chunk when `one_row`; otherwise it is looked up per element.
-struct RowCtx {
-  float mu, rf, oldsc, newsc, m128, m128n;
-  double rnew;
-  bool fast;
-};
-
-// A row value read once per row: wave-uniform (a scalar) when the wave works
-// on one row at a time, per lane when it packs several rows.
-template <bool PK>
-__device__ __forceinline__ float row_val(float x) {
-  return PK ? x : uniform_f(x);
-}
-
-// The rows of a wave's share of a slice, phases 5 and 6, in one of three
-// layouts.  LAY 0: one row at a time, lane l taking chunks l, l+64, ....
-// LAY 1 (rows of at most 32 chunks): L = 2^ceil(log2(chunks)) lanes per row,
-// 64 / L rows side by side, lane cl of a row's lane group taking chunk cl.
-// LAY 2 (an item of one row, e.g. a 1-D tensor): the four waves share the row,
-// wave w taking the chunk rounds w, w+4, ... of LAY 0.  Every element's
-// arithmetic is the same in all three; the only reductions across lanes are
-// the keep count (an integer sum), the int8 row absmax and the 4-bit block
-// absmax (maxima; blocks that cross chunks go through atomicMax), none of
-// which depends on the order.  Returns the lane's keep count.
-template <int OPT, int PHASE, int PT, int GT, int CODEC, int LAY>
-__device__ __forceinline__ uint32_t elem_rows(const KaonTensor& T, const KaonItem& it, const Ws& ws,
-                                              const KaonHyper& hp) {
-  const int64_t C = T.C, n = T.n;
-  const int64_t nch = (C + 7) >> 3;
-  const int cpl = (int)((nch + 63) >> 6);
-  const bool vec_t = T.vec_rows != 0;
-  const bool factored = T.factored != 0;
-  const bool gc = (hp.flags & KAON_F_GC) && factored;
-  const bool cautious = (hp.flags & KAON_F_CAUTIOUS) != 0;
-  const bool wd = (hp.flags & KAON_F_WD) != 0;
-  constexpr bool MUON = OPT == KAON_OPT_ADAMUON;
-  constexpr bool QUANT_C = CODEC == KAON_MOM_INT8 || CODEC == KAON_MOM_4BIT;
-  // AdaMuon's momentum is the raw grad's: float codecs were stored by the
-  // momentum pass; int8 / 4-bit codes are requantized here in phase 6
-  const bool mom = (hp.flags & KAON_F_MOMENTUM) != 0 && CODEC != KAON_MOM_NONE && (!MUON || (PHASE == 6 && QUANT_C));
-  const bool nk_remove = OPT == KAON_OPT_ADAKAON && mom && (hp.flags & KAON_F_NK_REMOVE);
-  const bool nk_climb = OPT == KAON_OPT_ADAKAON && mom && (hp.flags & KAON_F_NK_CLIMB);
-  const float nf_old = msam_nanfill(hp.nk_bound_old), nf_new = msam_nanfill(hp.nk_bound_new);
-  constexpr bool QUANT = CODEC == KAON_MOM_INT8 || CODEC == KAON_MOM_4BIT;
-  const bool quant = mom && QUANT;
-  const bool lowp = PT == KAON_BF16;
-  const int64_t B = CODEC == KAON_MOM_4BIT ? (int64_t)T.block4 : 1;
-  const int64_t nb = CODEC == KAON_MOM_4BIT ? nblocks4(T) : 0;
-  const WaveRows wr = wave_rows(it);
-
-  // clip divisor of the tensor (phase 4)
-  const float fac = OPT != KAON_OPT_LION ? ws.scal(T)[0] : 1.0f;
-  const double rfac = rcp64(fac);
-  double rden = 1.0;
-  if (PHASE == 6 && cautious) {
-    const uint32_t cnt = ((const KAON_G uint32_t*)ws.scal(T))[1];
-    rden = rcp64(fmaxf((float)cnt / (float)n, 1e-8f));
-  }
-  // 4-bit fast path: blocks inside rows, a block = G consecutive chunks = G lanes
-  const int64_t GL = CODEC == KAON_MOM_4BIT && B >= 8 ? B / 8 : 1;
-  const bool blk_fast = CODEC == KAON_MOM_4BIT && B % 8 == 0 && C % B == 0 && GL <= 64 && (64 % GL) == 0 && vec_t;
-  uint32_t keep = 0;
-  BlkMax bm4;  // 4-bit blocks across chunks or rows (phase 5)
-  // the scales of the last 4-bit block visited (blocks across chunks or rows):
-  // read once per run of a block's elements
-  uint32_t c_blk = 0xFFFFFFFFu;
-  float c_old = 1.0f, c_new = 1.0f;
-  double c_r = 1.0;
-  // lanes per row (2^lsh) and rows side by side (P); the lane's row in a pass
-  // and its chunk
-  constexpr bool PK = LAY == 1;
-  const int lsh = PK ? (nch <= 1 ? 0 : 32 - __builtin_clz((uint32_t)(nch - 1))) : 6;
-  const int P = 64 >> lsh;
-  const int grp = wr.lane >> lsh;
-  const int cl = wr.lane & ((1 << lsh) - 1);
-  // the lane that stores the row's values (LAY 2: of wave 0)
-  const bool lead = cl == 0 && (LAY != 2 || wr.w == 0);
-  // the rows and the chunk rounds of this wave
-  const int64_t rbeg = LAY == 2 ? (int64_t)it.row0 : wr.rb;
-  const int64_t rend = LAY == 2 ? (int64_t)it.row0 + 1 : wr.re;
-  const int k0 = LAY == 2 ? wr.w : 0;
-  constexpr int kstep = LAY == 2 ? 4 : 1;
-
-  for (int64_t r0 = rbeg; r0 < rend; r0 += P) {
-    // the lane's row; lanes past the wave's rows read the first row's context
-    // and take no chunk
-    const bool rvalid = r0 + grp < rend;
-    const int64_t r = rvalid ? r0 + grp : rbeg;
-    // ---- per-row context (wave-uniform unless PK)
-    RowCtx rc;
-    rc.mu = gc ? row_val<PK>(ws.mu(T)[r]) : 0.0f;
-    rc.rf = (OPT != KAON_OPT_LION && factored) ? row_val<PK>(ws.rf(T)[r]) : 0.0f;
-    rc.oldsc = 1.0f;
-    rc.newsc = 1.0f;
-    rc.rnew = 1.0;
-    if (CODEC == KAON_MOM_INT8 && mom) {
-      rc.oldsc = row_val<PK>(PHASE == 5 ? T.m_scale[r] : ws.roldsc(T)[r]);
-      if (PHASE == 6) {
-        rc.newsc = row_val<PK>(fmaxf(__uint_as_float(ws.ramax(T)[r]), 1e-12f) / 127.0f);
-        rc.rnew = rcp64(rc.newsc);
-      }
-    }
-    rc.fast = fabsf(rc.oldsc) < 0x1p120f && fabsf(rc.newsc) < 0x1p120f;
-    rc.m128 = -128.0f * rc.oldsc;
-    float row_amax = 0.0f;
-
-    for (int k = k0; k < cpl; k += kstep) {
-      const int64_t c = cl + 64 * k;
-      const int cnt = rvalid ? chunk_cnt(c, C) : 0;
-      const int64_t j0 = c * 8;
-      const int64_t e0 = r * C + j0;
-      const bool vec = vec_t && cnt == 8;
-      // ---- loads
-      float g[8], p[8], f[8];
-      uint32_t mq[8], pb[8];
-      if (cnt > 0) {
-        ld8<GT>(T.g, e0, cnt, vec, g);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) g[i] = 0.0f;
-      }
-      const bool need_p = PHASE == 6 || wd;
-      if (need_p && cnt > 0) {
-        if (PT != KAON_F32) {
-          ld8_bits(T.p, e0, cnt, vec, pb);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) p[i] = lp2f<PT>(pb[i]);
-        } else {
-          ld8<KAON_F32>(T.p, e0, cnt, vec, p);
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) p[i] = 0.0f;
-      }
-      if (mom && cnt > 0) ld_mom_raw<CODEC>(T, e0, cnt, vec, mq);
-      else
-#pragma unroll
-        for (int i = 0; i < 8; ++i) mq[i] = CODEC == KAON_MOM_4BIT ? 8u : 0u;
-      float ov[8];
-      if (MUON && cnt > 0) ld8<KAON_BF16>(ws.mo(T), e0, cnt, vec, ov);
-      if (OPT != KAON_OPT_LION && cnt > 0) {
-        if (factored) ld8<KAON_F32>((const float*)ws.cf(T), j0, cnt, vec, f);
-        else ld8<KAON_F32>(T.v, j0, cnt, vec, f);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] = 1.0f;
-      }
-      // 4-bit block scales: one block per chunk on the fast path
-      float b_old = 1.0f, b_new = 1.0f;
-      double b_rnew = 1.0;
-      int64_t blk = 0;
-      if (CODEC == KAON_MOM_4BIT && mom && blk_fast) {
-        blk = e0 / B;
-        if (cnt > 0) {
-          b_old = PHASE == 5 ? T.m_scale[blk] : ws.boldsc(T, nb)[blk];
-          if (PHASE == 6) {
-            b_new = fmaxf(__uint_as_float(ws.bamax(T)[blk]), 1e-12f) / 7.0f;
-            b_rnew = rcp64(b_new);
-          }
-        }
-      }
-      // ---- noise (phase 6, bf16 weights)
-      uint32_t nz0[8], nz1[8], nz2[8];
-      if (lowp && cnt > 0) {
-        const bool aligned = (e0 & 7) == 0;
-        if (nk_remove && need_p) {
-          if (aligned) noise8(hp.seed, hp.step, (uint32_t)T.tensor_id, 0u, e0, T.noise[0], cnt, nz0);
-          else
-#pragma unroll
-            for (int i = 0; i < 8; ++i) nz0[i] = i < cnt ? noise1(hp.seed, hp.step, T.tensor_id, 0u, e0 + i, T.noise[0]) : 0u;
-        }
-        if (PHASE == 6 && hp.bf16_method == KAON_SR) {
-          if (aligned) noise8(hp.seed, hp.step, (uint32_t)T.tensor_id, 1u, e0, T.noise[1], cnt, nz1);
-          else
-#pragma unroll
-            for (int i = 0; i < 8; ++i) nz1[i] = i < cnt ? noise1(hp.seed, hp.step, T.tensor_id, 1u, e0 + i, T.noise[1]) : 0u;
-        }
-        if (PHASE == 6 && nk_climb) {
-          if (aligned) noise8(hp.seed, hp.step, (uint32_t)T.tensor_id, 2u, e0, T.noise[2], cnt, nz2);
-          else
-#pragma unroll
-            for (int i = 0; i < 8; ++i) nz2[i] = i < cnt ? noise1(hp.seed, hp.step, T.tensor_id, 2u, e0 + i, T.noise[2]) : 0u;
-        }
-      }
-      // ---- gradient as the step sees it (GC in the grad dtype)
-      if (gc) {
-#pragma unroll
-        for (int i = 0; i < 8; i += 2) {
-          float a0 = g[i] - rc.mu, a1 = g[i + 1] - rc.mu;
-          round_pair<GT>(a0, a1);
-          g[i] = a0;
-          g[i + 1] = a1;
-        }
-      }
-      // ---- per element
-      uint32_t qout[8];
-      float dout[8], mnew[8];
-      float chunk_amax = 0.0f;
-      // 4-bit blocks that cross chunks or rows: the chunk's first block and offset
-      // (one 32-bit division, n < 2^32), then walked element by element
-      uint32_t wblk = 0u, woff = 0u;
-      if (CODEC == KAON_MOM_4BIT && mom && !blk_fast) {
-        wblk = (uint32_t)e0 / (uint32_t)B;
-        woff = (uint32_t)e0 - wblk * (uint32_t)B;
-      }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        qout[i] = mq[i];
-        dout[i] = 0.0f;
-        mnew[i] = 0.0f;
-        if (i >= cnt) continue;
-        float sc4_old = b_old, sc4_new = b_new;
-        double r4 = b_rnew;
-        int64_t blk_e = blk;
-        bool blk_first = false;  // the element opens its block
-        if (CODEC == KAON_MOM_4BIT && mom && !blk_fast) {
-          blk_e = wblk;
-          blk_first = woff == 0u;
-          if (++woff == (uint32_t)B) {
-            woff = 0u;
-            ++wblk;
-          }
-          if ((uint32_t)blk_e != c_blk) {
-            c_blk = (uint32_t)blk_e;
-            c_old = PHASE == 5 ? T.m_scale[blk_e] : ws.boldsc(T, nb)[blk_e];
-            if (PHASE == 6) {
-              c_new = fmaxf(__uint_as_float(ws.bamax(T)[blk_e]), 1e-12f) / 7.0f;
-              c_r = rcp64(c_new);
-            }
-          }
-          sc4_old = c_old;
-          sc4_new = c_new;
-          r4 = c_r;
-        }
-        float mold = 0.0f;
-        if (mom) {
-          if (CODEC == KAON_MOM_INT8) mold = dq_int8(mq[i], rc.oldsc, rc.m128, rc.fast);
-          else if (CODEC == KAON_MOM_4BIT) mold = ((float)mq[i] - 8.0f) * sc4_old;
-          else if (CODEC == KAON_MOM_BF16) mold = bf2f(mq[i]);
-          else if (CODEC == KAON_MOM_F32) mold = __uint_as_float(mq[i]);
-        }
-        float pw = p[i];  // weight the inner step sees (after the Nekaon removal)
-        if (nk_remove && need_p) {
-          const float ev = msam_e(mold * hp.nk_k, hp.nk_bound_old, nf_old);
-          pw = lowp ? bf2f(sr_bf16(p[i] + ev, nz0[i])) : p[i] + ev;
-        }
-        float d, mfv = 0.0f;
-        const float gv = g[i];
-        if (OPT == KAON_OPT_ADAKAON) {
-          const float u = factored ? (gv * rc.rf) * f[i] : gv * (1.0f / sqrtf(f[i]));
-          const float ud = (fac == 1.0f ? u : div_r64(u, rfac)) * hp.lr;
-          if (mom) {
-            if (CODEC == KAON_MOM_BF16) {
-              const uint32_t mb = f2bf(klerp(mold, rbf(ud), hp.w1));
-              qout[i] = mb;
-              d = bf2f(mb);
-            } else {
-              mfv = klerp(mold, ud, hp.w1);
-              d = mfv;
-              if (CODEC == KAON_MOM_F32) qout[i] = __float_as_uint(mfv);
-            }
-          } else {
-            d = ud;
-          }
-          if (wd) d = __fmaf_rn(hp.wdl, pw, d);
-        } else if (MUON) {
-          // U = O * r * c, clipped, times 0.2*lr (hp.lr); the momentum update
-          // is of the grad (requantized below)
-          const float u = (ov[i] * rc.rf) * f[i];
-          d = (fac == 1.0f ? u : div_r64(u, rfac)) * hp.lr;
-          if (mom) mfv = klerp(mold, gv, hp.w1);
-          if (wd) d = __fmaf_rn(hp.wdl, pw, d);
-        } else {  // Lion
-          const float cdir = __fmaf_rn(hp.a1, gv, mold * hp.b1);
-          d = ksign(cdir);
-          mfv = __fmaf_rn(hp.a2, gv, mold * hp.b2);
-          if (CODEC == KAON_MOM_F32) qout[i] = __float_as_uint(mfv);
-          else if (CODEC == KAON_MOM_BF16) qout[i] = f2bf(mfv);
-          if (wd) d = __fmaf_rn(hp.wdl, pw, d);
-        }
-        const bool kp = d * gv > 0.0f;
-        if (PHASE == 5) {
-          keep += kp ? 1u : 0u;
-          if (quant) {
-            const float ax = fabsf(mfv);
-            if (CODEC == KAON_MOM_4BIT && !blk_fast) {
-              bm4.add(ws.bamax(T), (uint32_t)blk_e, ax);
-              if (blk_first) ws.boldsc(T, nb)[blk_e] = sc4_old;
-            } else {
-              chunk_amax = fmaxf(chunk_amax, ax);
-            }
-          }
-        } else {
-          float mdeq = 0.0f;
-          if (quant) {
-            if (CODEC == KAON_MOM_INT8) {
-              float x = rintf(div_r64(mfv, rc.rnew));
-              x = fminf(fmaxf(x, -127.0f), 127.0f);
-              qout[i] = (uint32_t)(uint8_t)(int8_t)x;
-              mdeq = x * rc.newsc;
-            } else {
-              float x = rintf(div_r64(mfv, r4));
-              x = fminf(fmaxf(x, -7.0f), 7.0f);
-              qout[i] = (uint32_t)((int)x + 8);
-              mdeq = x * sc4_new;
-              if (!blk_fast && blk_first) T.m_scale[blk_e] = sc4_new;
-            }
-          } else if (mom) {
-            mdeq = CODEC == KAON_MOM_BF16 ? bf2f(qout[i]) : __uint_as_float(qout[i]);
-          }
-          mnew[i] = mdeq;
-          float dd = d;
-          if (cautious) dd = div_r64(d * (kp ? 1.0f : 0.0f), rden);
-          if (OPT == KAON_OPT_LION) dd = dd * hp.lr;
-          dout[i] = dd;
-          p[i] = pw;
-        }
-      }
-
-      if (PHASE == 5) {
-        if (quant && !(CODEC == KAON_MOM_4BIT && !blk_fast)) {
-          if (CODEC == KAON_MOM_INT8) {
-            row_amax = fmaxf(row_amax, chunk_amax);
-          } else {
-            // blocks of G lanes: reduce within the lane group, its first lane stores
-            float a = chunk_amax;
-            for (int o = (int)GL / 2; o >= 1; o >>= 1) a = fmaxf(a, __shfl_xor(a, o, 64));
-            if (cnt > 0 && (wr.lane % GL) == 0) {
-              ws.bamax(T)[blk] = __float_as_uint(a);
-              ws.boldsc(T, nb)[blk] = b_old;
-            }
-          }
-        }
-        continue;
-      }
-      if (cnt <= 0) continue;
-      // ---------------- phase 6 writes
-      if (gc && (hp.flags & KAON_F_GC_WRITE) && T.gc_write && (OPT == KAON_OPT_ADAKAON || OPT == KAON_OPT_LION)) {
-        // the centralized gradient over p.grad (already rounded to the grad dtype)
-        if (GT == KAON_F32) {
-          st8_f32(const_cast<void*>(T.g), e0, cnt, vec, g);
-        } else {
-          uint32_t gb[8];
-#pragma unroll
-          for (int i = 0; i < 8; ++i) gb[i] = f2lp<GT>(g[i]);
-          st8_bits(const_cast<void*>(T.g), e0, cnt, vec, gb);
-        }
-      }
-      if (CODEC == KAON_MOM_4BIT && mom && blk_fast && (wr.lane % GL) == 0) G(T.m_scale)[blk] = b_new;
-      if (mom) st_mom_raw<CODEC>(T, e0, cnt, vec, qout);
-      if (PT == KAON_F32) {
-        float o[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          float x = p[i] - dout[i];
-          if (nk_climb) x = x + msam_e(mnew[i] * (-hp.nk_k), hp.nk_bound_new, nf_new);
-          o[i] = x;
-        }
-        st8_f32(T.p, e0, cnt, vec, o);
-      } else {
-        uint32_t o[8];
-        if (hp.bf16_method == KAON_KAHAN) {
-          uint32_t sh[8];
-          ld8_bits(T.shift, e0, cnt, vec, sh);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            // shift -= lp(delta); p0 = p; p += shift; shift += p0 - p, in the
-            // param dtype (_backend.py:90-94)
-            const float s = round_to<PT>(lp2f<PT>(sh[i]) - round_to<PT>(dout[i]));
-            const float p0 = p[i];
-            const float p1 = round_to<PT>(p0 + s);
-            o[i] = f2lp<PT>(p1);
-            sh[i] = f2lp<PT>(s + round_to<PT>(p0 - p1));
-          }
-          st8_bits(T.shift, e0, cnt, vec, sh);
-        } else if (hp.bf16_method == KAON_RN || PT == KAON_F16) {
-          // fp16 params are written by RN under "stochastic_rounding" too: the
-          // reference's SR write is bf16-only (_backend.py:95-98)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) o[i] = f2lp<PT>(p[i] - round_to<PT>(dout[i]));
-        } else {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) o[i] = sr_bf16(p[i] - dout[i], nz1[i]);
-        }
-        if (nk_climb) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            o[i] = sr_bf16(bf2f(o[i]) + msam_e(mnew[i] * (-hp.nk_k), hp.nk_bound_new, nf_new), nz2[i]);
-        }
-        st8_bits(T.p, e0, cnt, vec, o);
-      }
-    }
-    // ---- end of row
-    if (CODEC == KAON_MOM_INT8 && quant) {
-      if (PHASE == 5) {
-        float am;
-        if (PK) {
-          // the maximum over the row's lane group (the other lanes of a
-          // 64-lane row hold 0, which a maximum of |m| ignores)
-          am = row_amax;
-          for (int o = (1 << lsh) >> 1; o >= 1; o >>= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
-        } else {
-          am = wave_max(row_amax);
-          if (LAY == 2) {
-            // the four waves' maxima (every wave is here: the row is the item's)
-            __shared__ float wmax[4];
-            if (wr.lane == 0) wmax[wr.w] = am;
-            __syncthreads();
-            am = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-          }
-        }
-        if (rvalid && lead) {
-          ws.ramax(T)[r] = __float_as_uint(am);
-          ws.roldsc(T)[r] = rc.oldsc;
-        }
-      } else if (rvalid && lead) {
-        T.m_scale[r] = rc.newsc;
-      }
-    }
-  }
-
-  if (PHASE == 5 && CODEC == KAON_MOM_4BIT) bm4.flush(ws.bamax(T));
-  return keep;
-}
-
-template <int OPT, int PHASE, int PT, int GT, int CODEC>
-__global__ __launch_bounds__(KAON_WG) void k_elem(const KaonTensor* __restrict__ D,
-                                                  const KaonItem* __restrict__ items, Ws ws, KaonHyper hp) {
-  __shared__ uint32_t keep_s[4];
-  const KaonItem it = items[blockIdx.x];
-  const KaonTensor& T = D[it.tensor];
-  const bool cautious = (hp.flags & KAON_F_CAUTIOUS) != 0;
-  uint32_t keep;
-  // rows of at most 32 chunks side by side (4-bit blocks are walked row by
-  // row); an item of one row over the four waves; otherwise a row per wave
-  bool done = false;
-  if constexpr (CODEC != KAON_MOM_4BIT) {
-    if (((T.C + 7) >> 3) <= 32) {
-      keep = elem_rows<OPT, PHASE, PT, GT, CODEC, 1>(T, it, ws, hp);
-      done = true;
-    }
-  }
-  if (!done) {
-    if (it.nrows == 1) keep = elem_rows<OPT, PHASE, PT, GT, CODEC, 2>(T, it, ws, hp);
-    else keep = elem_rows<OPT, PHASE, PT, GT, CODEC, 0>(T, it, ws, hp);
-  }
-  if (PHASE == 5 && cautious) {
-    const uint32_t wsum = wave_sum_u32(keep);
-    const WaveRows wr = wave_rows(it);
-    if (wr.lane == 0) keep_s[wr.w] = wsum;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const uint32_t tot = keep_s[0] + keep_s[1] + keep_s[2] + keep_s[3];
-      if (tot) atomicAdd(ws.keep_ctr(T), tot);
-    }
-  }
-}
-
 // =============================================================== AdaPNM
 // Phases 3, 5 and 6 of AdaPNM (_step_one_param, adapnm.py:1209-1275), per
 // element with g the (centralized) gradient:
@@ -1693,69 +1234,45 @@ __global__ __launch_bounds__(KAON_WG) void k_elem(const KaonTensor* __restrict__
 // the cautious keep count of d * g > 0.  Phase 6: requantize or store m_pos',
 // write p after the decoupled decay p * (1 - lr*wd).  The negative buffer is
 // only read.  Odd steps take m as the positive buffer, even steps m2.
-template <int PHASE, int PT, int GT, int CODEC>
+template <int GT, int CODEC>
 __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ D,
                                                  const KaonItem* __restrict__ items, Ws ws, KaonHyper hp) {
-  __shared__ uint32_t keep_s[4];
-  KaonItem it;
-  if (PHASE == 3) {
-    const KaonItem run = items[blockIdx.x / KAON_RUN];
-    const int sl = (int)(blockIdx.x % KAON_RUN);
-    if (sl >= run_slices(run)) return;
-    it = slice_item(run, sl);
-  } else {
-    it = items[blockIdx.x];
-  }
+  const KaonItem run = items[blockIdx.x / KAON_RUN];
+  const int sl = (int)(blockIdx.x % KAON_RUN);
+  if (sl >= run_slices(run)) return;
+  const KaonItem it = slice_item(run, sl);
   const KaonTensor& T = D[it.tensor];
-  const int64_t C = T.C, n = T.n;
+  const int64_t C = T.C;
   const int64_t nch = (C + 7) >> 3;
   const int cpl = (int)((nch + 63) >> 6);
   const bool vec_t = T.vec_rows != 0;
   const bool factored = T.factored != 0;
   const bool gc = (hp.flags & KAON_F_GC) && factored;
-  const bool cautious = (hp.flags & KAON_F_CAUTIOUS) != 0;
-  const bool wd = (hp.flags & KAON_F_WD) != 0;
   const bool ams = (hp.flags & KAON_F_AMS) && !factored && T.max_v;
-  const bool lowp = PT == KAON_BF16;
   constexpr bool QUANT = CODEC == KAON_MOM_INT8 || CODEC == KAON_MOM_4BIT;
   const bool swap = (hp.step & 1u) == 0u;
-  void* mpos = swap ? T.m2 : T.m;
+  const void* mpos = swap ? T.m2 : T.m;
   const void* mneg = swap ? T.m : T.m2;
-  float* spos = swap ? T.m2_scale : T.m_scale;
+  const float* spos = swap ? T.m2_scale : T.m_scale;
   const float* sneg = swap ? T.m_scale : T.m2_scale;
   const int64_t B = CODEC == KAON_MOM_4BIT ? (int64_t)T.block4 : 1;
   const int64_t nb = CODEC == KAON_MOM_4BIT ? nblocks4(T) : 0;
   const WaveRows wr = wave_rows(it);
-  const float fac = PHASE == 3 ? 1.0f : ws.scal(T)[0];
-  const double rfac = rcp64(fac);
-  double rden = 1.0;
-  if (PHASE == 6 && cautious) {
-    const uint32_t cnt = ((const KAON_G uint32_t*)ws.scal(T))[1];
-    rden = rcp64(fmaxf((float)cnt / (float)n, 1e-8f));
-  }
   const float* fsrc = factored ? (const float*)ws.cf(T) : (ams ? T.max_v : T.v);
-  uint32_t keep = 0;
-  BlkMax bm4;  // 4-bit blocks across chunks or rows (phase 3)
+  BlkMax bm4;  // 4-bit blocks across chunks or rows
   // the scales of the last 4-bit block visited: read once per run of its elements
   uint32_t c_blk = 0xFFFFFFFFu;
-  float c_o = 1.0f, c_g = 1.0f, c_n = 1.0f;
-  double c_r = 1.0;
+  float c_o = 1.0f, c_g = 1.0f;
 
   for (int64_t r = wr.rb; r < wr.re; ++r) {
     const float mu = gc ? uniform_f(ws.mu(T)[r]) : 0.0f;
     const float rf = factored ? uniform_f(ws.rf(T)[r]) : 0.0f;
-    // int8 per-row scales (one for a 1-D tensor): the positive buffer's old one
-    // (phase 6: as phase 3 recorded it), its new one (phase 6), the negative one
+    // int8 per-row scales (one for a 1-D tensor) of the positive and the negative buffer
     const int64_t sr = factored ? r : 0;
-    float oldsc = 1.0f, newsc = 1.0f, negsc = 1.0f;
-    double rnew = 1.0;
+    float oldsc = 1.0f, negsc = 1.0f;
     if (CODEC == KAON_MOM_INT8) {
-      oldsc = uniform_f(PHASE == 6 ? ws.roldsc(T)[r] : G(spos)[sr]);
+      oldsc = uniform_f(G(spos)[sr]);
       negsc = uniform_f(G(sneg)[sr]);
-      if (PHASE == 6) {
-        newsc = uniform_f(fmaxf(__uint_as_float(ws.ramax(T)[r]), 1e-12f) / 127.0f);
-        rnew = rcp64(newsc);
-      }
     }
     const bool dqf = fabsf(oldsc) < 0x1p120f && fabsf(negsc) < 0x1p120f;
     const float m128o = -128.0f * oldsc, m128n = -128.0f * negsc;
@@ -1768,28 +1285,12 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
       const int64_t j0 = c * 8;
       const int64_t e0 = r * C + j0;
       const bool vec = vec_t && cnt == 8;
-      float g[8], f[8], p[8];
-      uint32_t mq[8], nq[8], pb[8];
+      float g[8], f[8];
+      uint32_t mq[8], nq[8];
       ld8<GT>(T.g, e0, cnt, vec, g);
       ld_mom_at<CODEC>(mpos, e0, cnt, vec, mq);
       ld_mom_at<CODEC>(mneg, e0, cnt, vec, nq);
       ld8<KAON_F32>(fsrc, j0, cnt, vec, f);
-      if (PHASE == 6) {
-        if (PT != KAON_F32) {
-          ld8_bits(T.p, e0, cnt, vec, pb);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) p[i] = lp2f<PT>(pb[i]);
-        } else {
-          ld8<KAON_F32>(T.p, e0, cnt, vec, p);
-        }
-      }
-      uint32_t nz[8];
-      if (PHASE == 6 && lowp && hp.bf16_method == KAON_SR) {
-        if ((e0 & 7) == 0) noise8(hp.seed, hp.step, (uint32_t)T.tensor_id, 1u, e0, T.noise[1], cnt, nz);
-        else
-#pragma unroll
-          for (int i = 0; i < 8; ++i) nz[i] = i < cnt ? noise1(hp.seed, hp.step, T.tensor_id, 1u, e0 + i, T.noise[1]) : 0u;
-      }
       if (gc) {
 #pragma unroll
         for (int i = 0; i < 8; i += 2) {
@@ -1799,8 +1300,6 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
           g[i + 1] = a1;
         }
       }
-      uint32_t qout[8];
-      float dout[8];
       // 4-bit: the chunk's first block and offset (one 32-bit division, n < 2^31),
       // then walked element by element
       uint32_t wblk = 0u, woff = 0u;
@@ -1810,14 +1309,10 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
       }
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        qout[i] = mq[i];
-        dout[i] = 0.0f;
         if (i >= cnt) continue;
         // 4-bit block scales of the element
         int64_t blk = 0;
         bool blk_first = false;  // the element opens its block
-        float sc4o = 1.0f, sc4n = 1.0f, sc4g = 1.0f;
-        double r4 = 1.0;
         if (CODEC == KAON_MOM_4BIT) {
           blk = wblk;
           blk_first = woff == 0u;
@@ -1827,25 +1322,17 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
           }
           if ((uint32_t)blk != c_blk) {
             c_blk = (uint32_t)blk;
-            c_o = PHASE == 6 ? ws.boldsc(T, nb)[blk] : G(spos)[blk];
+            c_o = G(spos)[blk];
             c_g = G(sneg)[blk];
-            if (PHASE == 6) {
-              c_n = fmaxf(__uint_as_float(ws.bamax(T)[blk]), 1e-12f) / 7.0f;
-              c_r = rcp64(c_n);
-            }
           }
-          sc4o = c_o;
-          sc4g = c_g;
-          sc4n = c_n;
-          r4 = c_r;
         }
         float mold, mng;
         if (CODEC == KAON_MOM_INT8) {
           mold = dq_int8(mq[i], oldsc, m128o, dqf);
           mng = dq_int8(nq[i], negsc, m128n, dqf);
         } else if (CODEC == KAON_MOM_4BIT) {
-          mold = ((float)mq[i] - 8.0f) * sc4o;
-          mng = ((float)nq[i] - 8.0f) * sc4g;
+          mold = ((float)mq[i] - 8.0f) * c_o;
+          mng = ((float)nq[i] - 8.0f) * c_g;
         } else if (CODEC == KAON_MOM_BF16) {
           mold = bf2f(mq[i]);
           mng = bf2f(nq[i]);
@@ -1853,112 +1340,38 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
           mold = __uint_as_float(mq[i]);
           mng = __uint_as_float(nq[i]);
         }
-        const float gv = g[i];
-        const float mfv = __fmaf_rn(hp.a1, gv, mold * hp.b1);
+        const float mfv = __fmaf_rn(hp.a1, g[i], mold * hp.b1);
         const float pn = __fmaf_rn(hp.pn_neg, mng, mfv * hp.pn_pos) * hp.pn_rnorm;
         const float u = factored ? pn * ((rf * f[i]) * hp.bc2) : pn / ((sqrtf(f[i] + 1e-15f) + hp.eps1) / hp.bc2);
-        if (PHASE == 3) {
-          ss = ss + u * u;
-          if (QUANT) {
-            const float ax = fabsf(mfv);
-            if (CODEC == KAON_MOM_INT8) {
-              row_amax = fmaxf(row_amax, ax);
-            } else {
-              bm4.add(ws.bamax(T), (uint32_t)blk, ax);
-              if (blk_first) ws.boldsc(T, nb)[blk] = sc4o;
-            }
+        ss = ss + u * u;
+        if (QUANT) {
+          const float ax = fabsf(mfv);
+          if (CODEC == KAON_MOM_INT8) {
+            row_amax = fmaxf(row_amax, ax);
+          } else {
+            bm4.add(ws.bamax(T), (uint32_t)blk, ax);
+            if (blk_first) ws.boldsc(T, nb)[blk] = c_o;
           }
-          continue;
         }
-        const float d = (fac == 1.0f ? u : div_r64(u, rfac)) * hp.lr;
-        const bool kp = d * gv > 0.0f;
-        if (PHASE == 5) {
-          keep += kp ? 1u : 0u;
-          continue;
-        }
-        if (CODEC == KAON_MOM_INT8) {
-          float x = rintf(div_r64(mfv, rnew));
-          x = fminf(fmaxf(x, -127.0f), 127.0f);
-          qout[i] = (uint32_t)(uint8_t)(int8_t)x;
-        } else if (CODEC == KAON_MOM_4BIT) {
-          float x = rintf(div_r64(mfv, r4));
-          x = fminf(fmaxf(x, -7.0f), 7.0f);
-          qout[i] = (uint32_t)((int)x + 8);
-          if (blk_first) G(spos)[blk] = sc4n;
-        } else if (CODEC == KAON_MOM_BF16) {
-          qout[i] = f2bf(mfv);
-        } else {
-          qout[i] = __float_as_uint(mfv);
-        }
-        dout[i] = cautious ? div_r64(d * (kp ? 1.0f : 0.0f), rden) : d;
-        // p.data.mul_(1 - lr*wd) in the param dtype (adapnm.py:1227-1228)
-        if (wd) p[i] = round_to<PT>(p[i] * hp.wdl);
-      }
-      if (PHASE != 6) continue;
-      // ---------------- phase 6 writes
-      st_mom_at<CODEC>(mpos, n, e0, cnt, vec, qout);
-      if (PT == KAON_F32) {
-        float o[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) o[i] = p[i] - dout[i];
-        st8_f32(T.p, e0, cnt, vec, o);
-      } else {
-        uint32_t o[8];
-        if (hp.bf16_method == KAON_KAHAN) {
-          uint32_t sh[8];
-          ld8_bits(T.shift, e0, cnt, vec, sh);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            // kahan in the param dtype (_backend.py:90-94)
-            const float s = round_to<PT>(lp2f<PT>(sh[i]) - round_to<PT>(dout[i]));
-            const float p0 = p[i];
-            const float p1 = round_to<PT>(p0 + s);
-            o[i] = f2lp<PT>(p1);
-            sh[i] = f2lp<PT>(s + round_to<PT>(p0 - p1));
-          }
-          st8_bits(T.shift, e0, cnt, vec, sh);
-        } else if (hp.bf16_method == KAON_RN || PT == KAON_F16) {
-          // fp16 params take RN under "stochastic_rounding" too (_backend.py:95-98)
-#pragma unroll
-          for (int i = 0; i < 8; ++i) o[i] = f2lp<PT>(p[i] - round_to<PT>(dout[i]));
-        } else {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) o[i] = sr_bf16(p[i] - dout[i], nz[i]);
-        }
-        st8_bits(T.p, e0, cnt, vec, o);
       }
     }
     // ---- end of row
-    if (PHASE == 3) {
-      const float s2 = wave_csum(ss);
-      if (CODEC == KAON_MOM_INT8) {
-        const float am = wave_max(row_amax);
-        if (wr.lane == 0) {
-          ws.ramax(T)[r] = __float_as_uint(am);
-          ws.roldsc(T)[r] = oldsc;
-        }
+    const float s2 = wave_csum(ss);
+    if (CODEC == KAON_MOM_INT8) {
+      const float am = wave_max(row_amax);
+      if (wr.lane == 0) {
+        ws.ramax(T)[r] = __float_as_uint(am);
+        ws.roldsc(T)[r] = oldsc;
       }
-      if (wr.lane == 0) ws.rs(T)[r] = s2;
-    } else if (PHASE == 6 && CODEC == KAON_MOM_INT8 && wr.lane == 0) {
-      G(spos)[sr] = newsc;
     }
+    if (wr.lane == 0) ws.rs(T)[r] = s2;
   }
-
-  if (PHASE == 3 && CODEC == KAON_MOM_4BIT) bm4.flush(ws.bamax(T));
-  if (PHASE == 5 && cautious) {
-    const uint32_t wsum = wave_sum_u32(keep);
-    if (wr.lane == 0) keep_s[wr.w] = wsum;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const uint32_t tot = keep_s[0] + keep_s[1] + keep_s[2] + keep_s[3];
-      if (tot) atomicAdd(ws.keep_ctr(T), tot);
-    }
-  }
+  if (CODEC == KAON_MOM_4BIT) bm4.flush(ws.bamax(T));
 }
 
 // AdaPNM phase 3 on row class 0 (factored, bf16 g, 16-byte rows with
 // C % 8 == 0, at most 4 chunks per lane) with int8 or bf16 momenta: the same
-// arithmetic and 64-lane row order as k_pnm<3>, with all loads of a group of
+// arithmetic and 64-lane row order as k_pnm, with all loads of a group of
 // GR rows (g and both momenta, every chunk of the lane) issued before the
 // group's arithmetic, and the per-row values read once per wave (one row per
 // lane, then read across lanes).  Addresses are clamped to valid rows and
@@ -3034,29 +2447,6 @@ __global__ __launch_bounds__(KAON_WG) void k_copy(const ku4* __restrict__ src_, 
 
 // ------------------------------------------------------------ dispatch tables
 
-template <int OPT, int PHASE, int PT, int GT>
-ElemFn elem_by_codec(int codec) {
-  switch (codec) {
-    case KAON_MOM_NONE: return k_elem<OPT, PHASE, PT, GT, KAON_MOM_NONE>;
-    case KAON_MOM_F32: return k_elem<OPT, PHASE, PT, GT, KAON_MOM_F32>;
-    case KAON_MOM_BF16: return k_elem<OPT, PHASE, PT, GT, KAON_MOM_BF16>;
-    case KAON_MOM_INT8: return k_elem<OPT, PHASE, PT, GT, KAON_MOM_INT8>;
-    case KAON_MOM_4BIT: return k_elem<OPT, PHASE, PT, GT, KAON_MOM_4BIT>;
-  }
-  return nullptr;
-}
-
-template <int OPT, int PHASE>
-ElemFn elem_fn(int pt, int gt, int codec) {
-  if (pt == KAON_BF16 && gt == KAON_BF16) return elem_by_codec<OPT, PHASE, KAON_BF16, KAON_BF16>(codec);
-  if (pt == KAON_BF16 && gt == KAON_F32) return elem_by_codec<OPT, PHASE, KAON_BF16, KAON_F32>(codec);
-  if (pt == KAON_F32 && gt == KAON_BF16) return elem_by_codec<OPT, PHASE, KAON_F32, KAON_BF16>(codec);
-  if (pt == KAON_F32 && gt == KAON_F32) return elem_by_codec<OPT, PHASE, KAON_F32, KAON_F32>(codec);
-  if constexpr (OPT == KAON_OPT_ADAKAON || OPT == KAON_OPT_LION || OPT == KAON_OPT_ADAMUON)
-    if (pt == KAON_F16 && gt == KAON_F16) return elem_by_codec<OPT, PHASE, KAON_F16, KAON_F16>(codec);
-  return nullptr;
-}
-
 int fast_flags(const KaonHyper& h) {
   int ff = 0;
   if (h.flags & KAON_F_GC) ff |= FF_GC;
@@ -3069,7 +2459,7 @@ int fast_flags(const KaonHyper& h) {
 }
 
 // Phase 5 or 6 over the slices: the specialized kernel over elem_items[0,
-// n_fast) when one exists for the configuration, the generic one over the rest.
+// n_fast) when one exists for the configuration, the flat-chunk one over the rest.
 template <int OPT, int PHASE>
 int launch_elem(const KaonLaunch& L, Ws ws, const KaonHyper& h, int codec, hipStream_t st) {
   int32_t n_fast = L.n_fast;
@@ -3082,7 +2472,10 @@ int launch_elem(const KaonLaunch& L, Ws ws, const KaonHyper& h, int codec, hipSt
   }
   const int32_t rest = L.n_elem_items - n_fast;
   if (rest > 0) {
-    ElemFn fg = elem_fn<OPT, PHASE>(h.p_dtype, h.g_dtype, codec);
+    ElemFn fg = OPT == KAON_OPT_LION      ? (PHASE == 5 ? flat_lion5 : flat_lion6)(h, codec)
+                : OPT == KAON_OPT_ADAMUON ? (PHASE == 5 ? flat_muon5 : flat_muon6)(h, codec)
+                                          : (PHASE == 5 ? flat_ada5 : flat_ada6)(h, codec);
+    if (!fg) return fail("kaon: no keep-count / apply kernel for this dtype and codec combination");
     hipLaunchKernelGGL(fg, dim3(rest), dim3(KAON_WG), 0, st, L.descs, L.elem_items + n_fast, ws, h);
   }
   return check_launch(PHASE == 5 ? "kaon: keep-count launch" : "kaon: apply launch");
@@ -3164,24 +2557,19 @@ MuonMomFn muon_mom_gt(int codec) {
 }
 
 using PnmFn = void (*)(const KaonTensor*, const KaonItem*, Ws, KaonHyper);
-template <int PHASE, int PT, int GT>
+template <int GT>
 PnmFn pnm_by_codec(int codec) {
   switch (codec) {
-    case KAON_MOM_F32: return k_pnm<PHASE, PT, GT, KAON_MOM_F32>;
-    case KAON_MOM_BF16: return k_pnm<PHASE, PT, GT, KAON_MOM_BF16>;
-    case KAON_MOM_INT8: return k_pnm<PHASE, PT, GT, KAON_MOM_INT8>;
-    case KAON_MOM_4BIT: return k_pnm<PHASE, PT, GT, KAON_MOM_4BIT>;
+    case KAON_MOM_F32: return k_pnm<GT, KAON_MOM_F32>;
+    case KAON_MOM_BF16: return k_pnm<GT, KAON_MOM_BF16>;
+    case KAON_MOM_INT8: return k_pnm<GT, KAON_MOM_INT8>;
+    case KAON_MOM_4BIT: return k_pnm<GT, KAON_MOM_4BIT>;
   }
   return nullptr;
 }
-template <int PHASE>
 PnmFn pnm_fn(int pt, int gt, int codec) {
-  if (pt == KAON_BF16 && gt == KAON_BF16) return pnm_by_codec<PHASE, KAON_BF16, KAON_BF16>(codec);
-  if (pt == KAON_BF16 && gt == KAON_F32) return pnm_by_codec<PHASE, KAON_BF16, KAON_F32>(codec);
-  if (pt == KAON_F32 && gt == KAON_BF16) return pnm_by_codec<PHASE, KAON_F32, KAON_BF16>(codec);
-  if (pt == KAON_F32 && gt == KAON_F32) return pnm_by_codec<PHASE, KAON_F32, KAON_F32>(codec);
-  if (pt == KAON_F16 && gt == KAON_F16) return pnm_by_codec<PHASE, KAON_F16, KAON_F16>(codec);
-  return nullptr;
+  if (pt == KAON_F16 || gt == KAON_F16) return pt == gt ? pnm_by_codec<KAON_F16>(codec) : nullptr;
+  return gt == KAON_BF16 ? pnm_by_codec<KAON_BF16>(codec) : pnm_by_codec<KAON_F32>(codec);
 }
 
 using PdFn = void (*)(const KaonTensor*, const KaonItem*, Ws, KaonHyper);
@@ -3478,9 +2866,9 @@ int kaon_adapnm_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask, 
   KaonHyper h = *hp;
   h.flags |= KAON_F_PNM | KAON_F_MOMENTUM;
   h.flags &= ~(KAON_F_NK_REMOVE | KAON_F_NK_CLIMB | KAON_F_SRC_O);
-  PnmFn f3 = pnm_fn<3>(h.p_dtype, h.g_dtype, h.codec);
-  PnmFn f5 = pnm_fn<5>(h.p_dtype, h.g_dtype, h.codec);
-  PnmFn f6 = pnm_fn<6>(h.p_dtype, h.g_dtype, h.codec);
+  PnmFn f3 = pnm_fn(h.p_dtype, h.g_dtype, h.codec);
+  ElemFn f5 = flat_pnm5(h, h.codec);
+  ElemFn f6 = flat_pnm6(h, h.codec);
   if (!f3 || !f5 || !f6) return fail("kaon_adapnm_step: unsupported dtype / codec combination");
   if (mask & (1u << 1)) {
     if ((rc = launch_stats(*L, ws, h, 0, st))) return rc;
@@ -3508,10 +2896,10 @@ int kaon_adapnm_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask, 
     if ((rc = check_launch("kaon: k_clipdiv launch"))) return rc;
   }
   // phases 5 and 6: the specialized kernel over the fast slices when one exists
-  // for the configuration, the generic one over the rest
+  // for the configuration, the flat-chunk one over the rest
   const bool fast_cfg = L->n_fast > 0 && h.bf16_method == KAON_SR && h.p_dtype == KAON_BF16 &&
                         h.g_dtype == KAON_BF16;
-  auto launch_pnm = [&](ElemFn ff, PnmFn fg, const char* what) {
+  auto launch_pnm = [&](ElemFn ff, ElemFn fg, const char* what) {
     const int32_t n_fast = ff ? L->n_fast : 0;
     if (n_fast > 0)
       hipLaunchKernelGGL(ff, dim3(n_fast), dim3(KAON_WG), 0, st, L->descs, L->elem_items, ws, h);

@@ -336,7 +336,7 @@ __device__ __forceinline__ void tfin_cols(const KaonTensor& T, const Ws& ws, con
     const int64_t j = j0 + c;
     const float nc = klerp(G(T.col)[j], cs[c] / (float)R, hp.w2);
     G(T.col)[j] = nc;
-    ws.cf(T)[j] = 1.0f / sqrtf(nc);
+    put_cf(ws.cf(T), T.C, j, 1.0f / sqrtf(nc));
   }
 }
 
@@ -367,7 +367,7 @@ __device__ void tfin_scalar(const KaonTensor& T, const Ws& ws, const KaonHyper& 
     }
     const float nc = klerp(G(T.col)[j], cs / (float)R, hp.w2);
     G(T.col)[j] = nc;
-    ws.cf(T)[j] = 1.0f / sqrtf(nc);
+    put_cf(ws.cf(T), T.C, j, 1.0f / sqrtf(nc));
   }
 }
 
