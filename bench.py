@@ -154,7 +154,7 @@ def phase_bytes(phase: int, bm: float, wd: bool, opt: str = "adakaon", w: dict |
 
 
 KERNEL_SOURCES = ("k-optimizers_amd/csrc/kaon_step.hip", "k-optimizers_amd/csrc/kaon_fast.hip",
-                  "k-optimizers_amd/csrc/kaon_flat.hip",
+                  "k-optimizers_amd/csrc/kaon_flat.hip", "k-optimizers_amd/csrc/kaon_stats.hip",
                   "k-optimizers_amd/csrc/kaon_common.h", "k-optimizers_amd/csrc/kaon_device.h",
                   "k-optimizers_amd/csrc/kaon_ns.hip", "k-optimizers_amd/csrc/kaon_plan.cpp")
 

@@ -259,6 +259,11 @@ int torch_momentum_sumsq(const KaonLaunch& L, Ws ws, int codec, hipStream_t st);
 // [t0, t1) (descs[k].by_size); a HIP status.
 int torch_clip(const KaonLaunch& L, Ws ws, const KaonHyper& h, int32_t t0, int32_t t1, hipStream_t st);
 
+// Phase 1 (kaon_stats.hip): the row statistics of every run, mode 0 (Adakaon,
+// AdaMuon, AdaPNM, KProdigy) or 1 (Lion: GC means only).  Returns the text of an
+// error, or nullptr.
+const char* launch_stats(const KaonLaunch& L, Ws ws, const KaonHyper& hp, int mode, hipStream_t st);
+
 // A phase-5/6 kernel over work items: (descriptors, items, workspace, hyper-parameters).
 using ElemFn = void (*)(const KaonTensor*, const KaonItem*, Ws, KaonHyper);
 

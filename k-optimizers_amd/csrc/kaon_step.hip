@@ -9,6 +9,8 @@
 //   writes   src/kaon/_backend.py:82-142, _stochastic_rounding.py:70-103
 //   factored src/kaon/_factored.py:26-83; GC src/kaon/_backend.py:147-177
 //
+// Phase 1 is in kaon_stats.hip, phases 5 and 6 in kaon_fast.hip and kaon_flat.hip.
+//
 // Work decomposition.  A work item is a slice: 4 wave groups of RW
 // consecutive rows of one tensor (RW = max(1, 20 / chunks-per-lane) so a wave
 // group spans about 160 elements per lane).  Each wave64 owns its rows whole:
@@ -60,453 +62,6 @@ int check_launch(const char* what) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return fail(what, e);
   return 0;
-}
-
-// Columns per LDS segment of the streamed rows' column fold (phase 1).
-constexpr int kSeg = 4096;
-
-// KProdigy's coupled decay folded into the gradient its second moment sees,
-// g' = fma(wd, p, GC(g)) (_collect_grad, kprodigy.py:406-414; torch's add with
-// alpha is one fused multiply-add), for the generic phase-1 kernel.
-__device__ __forceinline__ void add_coupled_wd(const KaonTensor& T, const KaonHyper& hp, int64_t e0, int cnt, bool vv,
-                                               float x[8]) {
-  float p[8];
-  if (hp.p_dtype == KAON_BF16) ld8<KAON_BF16>(T.p, e0, cnt, vv, p);
-  else if (hp.p_dtype == KAON_F16) ld8<KAON_F16>(T.p, e0, cnt, vv, p);
-  else ld8<KAON_F32>(T.p, e0, cnt, vv, p);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) x[i] = __fmaf_rn(hp.wdl, p[i], x[i]);
-}
-
-// =============================================================== phase 1
-// The canonical row sum of a row held by an aligned group of 2^lsh <= 32
-// lanes (lane cl of the group holding the sum of its chunk cl, 0 past the
-// row's chunks).  The 64-lane butterfly of the one-row-per-wave layout adds,
-// at offsets 32 ... 2^lsh, only the +0 of lanes past the row, which leaves each
-// lane sum x as x + 0 (-0 becomes +0); its offsets 2^(lsh-1) ... 1 pair lanes
-// of the same group.  So the sum is that group's butterfly of x + 0.
-__device__ __forceinline__ float group_csum(float a, int lsh) {
-  float v = a + 0.0f;
-  for (int o = (1 << lsh) >> 1; o >= 1; o >>= 1) v = v + __shfl_xor(v, o, 64);
-  return v;
-}
-
-// Phase 1 of one slice of a factored tensor whose rows have at most 32 chunks
-// (the register layouts, RW > 1 rows per wave group, no coupled decay).  A
-// wave works on 64 / L of its rows side by side, L = 2^ceil(log2(chunks))
-// lanes per row, lane cl of a row's group taking chunk cl: one memory round
-// trip per 64 / L rows instead of one per row.  Every value and every sum
-// order is that of k_stats's one-row-at-a-time body: the row sums through
-// group_csum, and each column partial (the wave group's rows added in row
-// order, then the wave groups folded in order in LDS) built by lane group 0,
-// which takes each row's values from that row's lane group in turn.
-template <int GT>
-__device__ __forceinline__ void stats_packed(const KaonTensor& T, const KaonItem& sit, const Ws& ws,
-                                             const KaonHyper& hp, int mode, const void* gsrc, KAON_G float* part,
-                                             KAON_G float* part2, bool first, bool alg, float* lds_col) {
-  const int64_t C = T.C;
-  const int nch = (int)((C + 7) >> 3);
-  const bool vec = T.vec_rows != 0;
-  const bool eps = (hp.flags & KAON_F_EPS) != 0;
-  const bool gc = (hp.flags & KAON_F_GC) != 0;
-  const WaveRows wr = wave_rows(sit);
-  const int lsh = nch <= 1 ? 0 : 32 - __builtin_clz((uint32_t)(nch - 1));
-  const int P = 64 >> lsh;
-  const int grp = wr.lane >> lsh;
-  const int cl = wr.lane & ((1 << lsh) - 1);
-  const int cnt0 = chunk_cnt(cl, C);  // elements of the lane's chunk in any row
-  KAON_G float* mu_arr = ws.mu(T);
-  float colacc[8], acc2[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    colacc[i] = 0.0f;
-    acc2[i] = 0.0f;
-  }
-  for (int64_t r0 = wr.rb; r0 < wr.re; r0 += P) {
-    const int nv = (int)min<int64_t>(P, wr.re - r0);  // rows of this pass (wave-uniform)
-    const bool rvalid = grp < nv;
-    const int64_t r = rvalid ? r0 + grp : wr.rb;
-    const int cnt = rvalid ? cnt0 : 0;
-    float x[8];
-    if (cnt > 0) {
-      ld8<GT>(gsrc, r * C + (int64_t)cl * 8, cnt, vec && cnt == 8, x);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) x[i] = 0.0f;
-    }
-    const float row_old = mode == 0 ? T.row[r] : 0.0f;
-    float xb[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) xb[i] = x[i];
-    float mu = 0.0f;
-    if (gc) {
-      float a = 0.0f;
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (i < cnt) a = a + x[i];
-      mu = round_to<GT>(group_csum(a, lsh) / (float)C);
-      if (rvalid && cl == 0) mu_arr[r] = mu;
-#pragma unroll
-      for (int i = 0; i < 8; i += 2) {
-        float a0 = xb[i] - mu, a1 = xb[i + 1] - mu;
-        round_pair<GT>(a0, a1);
-        xb[i] = a0;
-        xb[i + 1] = a1;
-      }
-    }
-    if (mode == 1) continue;
-    float q[8];
-    float a2 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      q[i] = xb[i] * xb[i];
-      if (eps) q[i] = q[i] + hp.eps1;
-      if (i < cnt) a2 = a2 + q[i];
-    }
-    const float s2 = group_csum(a2, lsh);
-    const float nr = klerp(row_old, s2 / (float)C, hp.w2);
-    if (rvalid && cl == 0) T.row[r] = nr;
-    // the column partial: rows r0, r0 + 1, ... in order
-    for (int g = 0; g < nv; ++g) {
-      const int src = (g << lsh) + cl;
-#pragma unroll
-      for (int i = 0; i < 8; ++i) colacc[i] = colacc[i] + __shfl(q[i], src, 64);
-    }
-    if (alg) {
-      // the clip's second column partial, t = (G * G) / row (the new row; no
-      // eps1), G formed again from the raw gradient as the row-by-row body does
-      const float w = 1.0f / nr;
-      float t[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float gv = gc ? round_to<GT>(x[i] - mu) : x[i];
-        t[i] = (gv * gv) * w;
-      }
-      for (int g = 0; g < nv; ++g) {
-        const int src = (g << lsh) + cl;
-        const bool start = r0 == wr.rb && g == 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float tv = __shfl(t[i], src, 64);
-          acc2[i] = start ? tv : acc2[i] + tv;
-        }
-      }
-    }
-  }
-  if (mode == 1) return;
-  // fold the wave-group partials in group order into the slice partial (lane
-  // group 0 holds them, lane cl for chunk cl), then into the run partial
-  const bool has_rows = wr.re > wr.rb;
-  const bool holder = grp == 0 && has_rows;
-  for (int wf = 0; wf < 4; ++wf) {
-    if (wr.w == wf && holder) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (i < cnt0) {
-          const int j = cl * 8 + i;
-          lds_col[j] = wf == 0 ? colacc[i] : lds_col[j] + colacc[i];
-        }
-    }
-    __syncthreads();
-  }
-  for (int64_t j = threadIdx.x; j < C; j += KAON_WG) part[j] = first ? lds_col[j] : part[j] + lds_col[j];
-  __syncthreads();  // lds_col is reused
-  if (!alg) return;
-  for (int wf = 0; wf < 4; ++wf) {
-    if (wr.w == wf && holder) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (i < cnt0) {
-          const int j = cl * 8 + i;
-          lds_col[j] = wf == 0 ? acc2[i] : lds_col[j] + acc2[i];
-        }
-    }
-    __syncthreads();
-  }
-  for (int64_t j = threadIdx.x; j < C; j += KAON_WG) part2[j] = first ? lds_col[j] : part2[j] + lds_col[j];
-  __syncthreads();  // lds_col is reused by the next slice
-}
-
-// mode 0 (Adakaon): GC row mean (stored), row EMA of mean_C(G^2), column
-// partial of the slice (wave groups folded in order in LDS); 1-D tensors: v
-// EMA.  mode 1 (Lion): GC row means only.  CPL > 0 keeps a row of up to CPL
-// chunks per lane in registers; CPL == 0 streams the row from memory (used for
-// rows longer than 24 chunks per lane, fp32 grads with long rows, and 1-D).
-// With KAON_F_PD_COUPLED (KProdigy, factored, coupled decay) G is the decayed
-// gradient fma(wd, p, GC(g)); the GC mean is still the raw gradient's.
-template <int GT, int CPL>
-__global__ __launch_bounds__(KAON_WG) void k_stats(const KaonTensor* __restrict__ D,
-                                                   const KaonItem* __restrict__ items, Ws ws, KaonHyper hp,
-                                                   int mode) {
-  extern __shared__ float lds_col[];
-  __shared__ float winv_s[4][KAON_ROW_BUDGET];  // 1 / row (the new row) of each wave's rows
-  __shared__ float red4[4];
-  const KaonItem it = items[blockIdx.x];
-  const KaonTensor& T = D[it.tensor];
-  // KProdigy's per-element v and its block-factored tensors: their own pass 1 kernels
-  if (T.full_v || T.fb_r) return;
-  zero_accumulators(T, it, ws, hp.codec);
-  const void* gsrc = ws.src(T, hp.flags);
-  const int64_t C = T.C;
-  const int64_t nch = (C + 7) >> 3;
-  const int cpl = (int)((nch + 63) >> 6);
-  const bool vec = T.vec_rows != 0;
-  const bool eps = (hp.flags & KAON_F_EPS) != 0;
-  const bool alg = clip_alg(hp, mode);
-  const bool cwd = mode == 0 && (hp.flags & KAON_F_PD_COUPLED) != 0;
-
-  if (!T.factored) {
-    if (mode == 0) stats_1d<GT>(T, gsrc, hp, alg ? ws.scal(T) : nullptr, red4);
-    return;
-  }
-
-  const bool gc = (hp.flags & KAON_F_GC) != 0;
-  if (mode == 1 && !gc) return;
-  KAON_G float* mu_arr = ws.mu(T);
-  const int RW = it.kind;
-  KAON_G float* part = run_part(ws, T, it);
-  const int nsl = run_slices(it);
-  // rows of at most 32 chunks (the class of 1-4 chunks per lane): side by side
-  const bool packed = CPL == 4 && nch <= 32 && RW > 1 && !cwd;
-#pragma clang loop unroll(disable)
-  for (int sl = 0; sl < nsl; ++sl) {
-  if constexpr (CPL == 4) {
-    if (packed) {
-      stats_packed<GT>(T, slice_item(it, sl), ws, hp, mode, gsrc, part, part + (int64_t)T.ngroups * C, sl == 0, alg,
-                       lds_col);
-      continue;
-    }
-  }
-  const WaveRows wr = wave_rows(slice_item(it, sl));
-
-  // registers: row buffer (CPL chunks) and the wave-group column partial
-  constexpr int NB = CPL > 0 ? CPL : 1;
-  float xb[NB][8];
-  float colacc[NB][8];
-#pragma unroll
-  for (int k = 0; k < NB; ++k)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) colacc[k][i] = 0.0f;
-
-  for (int64_t r = wr.rb; r < wr.re; ++r) {
-    const int64_t rowoff = r * C;
-    float mu = 0.0f;
-    if (CPL > 0) {
-#pragma unroll
-      for (int k = 0; k < NB; ++k) {
-        const int64_t c = wr.lane + 64 * k;
-        const int cnt = k < cpl ? chunk_cnt(c, C) : 0;
-        if (cnt > 0) ld8<GT>(gsrc, rowoff + c * 8, cnt, vec && cnt == 8, xb[k]);
-        else
-#pragma unroll
-          for (int i = 0; i < 8; ++i) xb[k][i] = 0.0f;
-      }
-      if (gc) {
-        float a = 0.0f;
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-          const int cnt = k < cpl ? chunk_cnt(wr.lane + 64 * k, C) : 0;
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (i < cnt) a = a + xb[k][i];
-        }
-        mu = round_to<GT>(wave_csum(a) / (float)C);
-        if (wr.lane == 0) mu_arr[r] = mu;
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-#pragma unroll
-          for (int i = 0; i < 8; i += 2) {
-            float a0 = xb[k][i] - mu, a1 = xb[k][i + 1] - mu;
-            round_pair<GT>(a0, a1);
-            xb[k][i] = a0;
-            xb[k][i + 1] = a1;
-          }
-        }
-      }
-      if (mode == 1) continue;
-      if (cwd) {
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-          const int64_t c = wr.lane + 64 * k;
-          const int cnt = k < cpl ? chunk_cnt(c, C) : 0;
-          if (cnt > 0) add_coupled_wd(T, hp, rowoff + c * 8, cnt, vec && cnt == 8, xb[k]);
-        }
-      }
-      float a2 = 0.0f;
-#pragma unroll
-      for (int k = 0; k < NB; ++k) {
-        const int cnt = k < cpl ? chunk_cnt(wr.lane + 64 * k, C) : 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (i < cnt) {
-            float q = xb[k][i] * xb[k][i];
-            if (eps) q = q + hp.eps1;
-            a2 = a2 + q;
-            if (RW > 1) colacc[k][i] = colacc[k][i] + q;
-          }
-      }
-      const float s2 = wave_csum(a2);
-      const float nr = klerp(T.row[r], s2 / (float)C, hp.w2);
-      if (wr.lane == 0) {
-        T.row[r] = nr;
-        if (alg) winv_s[wr.w][r - wr.rb] = 1.0f / nr;
-      }
-    } else {
-      // streaming: sweep A (GC sum), sweep B (q and the row sum)
-      if (gc) {
-        float a = 0.0f;
-        for (int k = 0; k < cpl; ++k) {
-          const int64_t c = wr.lane + 64 * k;
-          const int cnt = chunk_cnt(c, C);
-          if (cnt <= 0) continue;
-          float x[8];
-          ld8<GT>(gsrc, rowoff + c * 8, cnt, vec && cnt == 8, x);
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (i < cnt) a = a + x[i];
-        }
-        mu = round_to<GT>(wave_csum(a) / (float)C);
-        if (wr.lane == 0) mu_arr[r] = mu;
-      }
-      if (mode == 1) continue;
-      float a2 = 0.0f;
-      for (int k = 0; k < cpl; ++k) {
-        const int64_t c = wr.lane + 64 * k;
-        const int cnt = chunk_cnt(c, C);
-        if (cnt <= 0) continue;
-        float x[8];
-        ld8<GT>(gsrc, rowoff + c * 8, cnt, vec && cnt == 8, x);
-        if (gc) {
-#pragma unroll
-          for (int i = 0; i < 8; ++i) x[i] = round_to<GT>(x[i] - mu);
-        }
-        if (cwd) add_coupled_wd(T, hp, rowoff + c * 8, cnt, vec && cnt == 8, x);
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (i < cnt) {
-            float q = x[i] * x[i];
-            if (eps) q = q + hp.eps1;
-            a2 = a2 + q;
-          }
-      }
-      const float s2 = wave_csum(a2);
-      const float nr = klerp(T.row[r], s2 / (float)C, hp.w2);
-      if (wr.lane == 0) {
-        T.row[r] = nr;
-        if (alg) winv_s[wr.w][r - wr.rb] = 1.0f / nr;
-      }
-    }
-  }
-  if (mode == 1) continue;
-
-  // fold the wave-group partials in group order into the slice partial
-  const bool has_rows = wr.re > wr.rb;
-  if (CPL == 0) {
-    // streamed rows (RW == 1, any length): the slice partial is folded kSeg
-    // columns at a time through LDS.  Per column the order is the one below:
-    // wave 0 + wave 1 + wave 2 + wave 3, then the slice added to the run partial.
-    for (int64_t c0 = 0; c0 < C; c0 += kSeg) {
-      const int64_t c1 = min(C, c0 + (int64_t)kSeg);
-      for (int wf = 0; wf < 4; ++wf) {
-        if (wr.w == wf && has_rows) {
-          const int64_t r = wr.rb;
-          const float mu = gc ? mu_arr[r] : 0.0f;
-          for (int64_t c = (c0 >> 3) + wr.lane; c * 8 < c1; c += 64) {
-            const int cnt = chunk_cnt(c, C);
-            float x[8];
-            ld8<GT>(gsrc, r * C + c * 8, cnt, vec && cnt == 8, x);
-            if (gc) {
-#pragma unroll
-              for (int i = 0; i < 8; ++i) x[i] = round_to<GT>(x[i] - mu);
-            }
-            if (cwd) add_coupled_wd(T, hp, r * C + c * 8, cnt, vec && cnt == 8, x);
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-              if (i < cnt) {
-                float v = x[i] * x[i];
-                if (eps) v = v + hp.eps1;
-                const int64_t j = c * 8 + i - c0;
-                lds_col[j] = wf == 0 ? v : lds_col[j] + v;
-              }
-          }
-        }
-        __syncthreads();
-      }
-      for (int64_t j = c0 + threadIdx.x; j < c1; j += KAON_WG)
-        part[j] = sl == 0 ? lds_col[j - c0] : part[j] + lds_col[j - c0];
-      __syncthreads();  // lds_col is reused by the next segment
-    }
-  } else {
-  for (int wf = 0; wf < 4; ++wf) {
-    if (wr.w == wf && has_rows) {
-      if (CPL > 0) {
-#pragma unroll
-        for (int k = 0; k < NB; ++k) {
-          const int64_t c = wr.lane + 64 * k;
-          const int cnt = k < cpl ? chunk_cnt(c, C) : 0;
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (i < cnt) {
-              float v;
-              if (RW > 1) {
-                v = colacc[k][i];
-              } else {
-                v = xb[k][i] * xb[k][i];
-                if (eps) v = v + hp.eps1;
-              }
-              const int64_t j = c * 8 + i;
-              lds_col[j] = wf == 0 ? v : lds_col[j] + v;
-            }
-        }
-      }
-    }
-    __syncthreads();
-  }
-  // the run partial: the slice partials added in slice order
-  for (int64_t j = threadIdx.x; j < C; j += KAON_WG) part[j] = sl == 0 ? lds_col[j] : part[j] + lds_col[j];
-  __syncthreads();  // lds_col is reused by the next slice
-  }
-  if (!alg) continue;
-  // The clip's second column partial, t = (G * G) / row (the new row; no
-  // eps1), in the same wave-group / slice / run order, the rows read again
-  // (this kernel serves the grad layouts outside the prefetching kernels'
-  // register budget).
-  KAON_G float* part2 = part + (int64_t)T.ngroups * C;
-  const int64_t segC = CPL > 0 ? C : (int64_t)kSeg;
-  for (int64_t c0 = 0; c0 < C; c0 += segC) {
-    const int64_t c1 = min(C, c0 + segC);
-    for (int wf = 0; wf < 4; ++wf) {
-      if (wr.w == wf && has_rows) {
-        for (int64_t c = (c0 >> 3) + wr.lane; c * 8 < c1; c += 64) {
-          const int cnt = chunk_cnt(c, C);
-          float acc[8];
-          for (int64_t r = wr.rb; r < wr.re; ++r) {
-            const float mu = gc ? mu_arr[r] : 0.0f;
-            const float w = winv_s[wf][r - wr.rb];
-            float x[8];
-            ld8<GT>(gsrc, r * C + c * 8, cnt, vec && cnt == 8, x);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              const float gv = gc ? round_to<GT>(x[i] - mu) : x[i];
-              const float t = (gv * gv) * w;
-              acc[i] = r == wr.rb ? t : acc[i] + t;
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < 8; ++i)
-            if (i < cnt) {
-              const int64_t j = c * 8 + i - c0;
-              lds_col[j] = wf == 0 ? acc[i] : lds_col[j] + acc[i];
-            }
-        }
-      }
-      __syncthreads();
-    }
-    for (int64_t j = c0 + threadIdx.x; j < c1; j += KAON_WG)
-      part2[j] = sl == 0 ? lds_col[j - c0] : part2[j] + lds_col[j - c0];
-    __syncthreads();  // lds_col is reused by the next segment or slice
-  }
-  }
 }
 
 // =============================================================== phase 2
@@ -612,352 +167,6 @@ __global__ __launch_bounds__(KAON_WG) void k_clipdiv(const KaonTensor* __restric
   // clip_threshold 0 (AdaPNM) leaves the update unclipped (adapnm.py:157-161)
   if (lane == 0) ws.scal(T)[0] = hp.clip > 0.0f ? fmaxf((sqrtf(ss) / T.sqrt_n) / hp.clip, 1.0f) : 1.0f;
 }
-
-// =============================================================== prefetching row kernels
-// Phase 1 for slices of bf16 grads with 16-byte rows (C % 8 == 0) of at
-// most 24 chunks per lane.  A wave loads its whole wave group (RW rows, RW *
-// CPL <= 24 chunks per lane) into registers as packed bf16 with every load
-// issued before the first use, so each lane keeps up to 24 x 16 bytes in
-// flight; the row reductions and the column fold then run from registers.
-// The arithmetic and its order are those of k_stats.
-
-// Chunk k of the lane in each of the wave group's rows.  Every load is
-// issued unconditionally from a valid address (rows past the group and
-// chunks past the row end load the last ones again, and a wave without rows
-// loads row `rsafe`), so no load waits behind a divergent branch; the caller
-// ignores the extra values.
-template <int CPL, int RW>
-__device__ __forceinline__ void load_group(const uint16_t* __restrict__ g, int64_t rb, int nrows, int64_t rsafe,
-                                           int64_t C, int nch, int lane, ku4 (&raw)[RW][CPL]) {
-  uint32_t off[CPL];
-#pragma unroll
-  for (int k = 0; k < CPL; ++k) off[k] = 16u * (uint32_t)min(lane + 64 * k, nch - 1);
-#pragma unroll
-  for (int j = 0; j < RW; ++j) {
-    const int64_t r = nrows > 0 ? rb + min(j, nrows - 1) : rsafe;
-    const KAON_G uint8_t* rowp = (const KAON_G uint8_t*)G(g + r * C);
-#pragma unroll
-    for (int k = 0; k < CPL; ++k) raw[j][k] = ld_stream<true>((const KAON_G ku4*)(rowp + off[k]));
-  }
-}
-
-// q = (G - mu)^2 (+ eps1) of one chunk, G - mu rounded to bf16 (GC in the
-// grad dtype).  EPS 0: no eps1; 2: x*x + eps1 rounded twice; 1: the same as
-// one fused multiply-add, which gives the same bits for every bf16-valued x
-// when eps1 is 0 or at least 2^-100: x*x is exact unless |x| < 2^-67, and
-// then x*x < 2^-134 lies below half an ulp of eps1, so both forms give eps1.
-// With gc the chunk's GC'd values replace it in `v` (bf16 pairs packed as
-// loaded), for the clip partial's second pass over the row registers.
-template <int EPS>
-__device__ __forceinline__ void sq_chunk(ku4& v, float mu, bool gc, float e1, float q[8]) {
-  float x[8];
-  if (gc) {
-    uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const float a0 = __uint_as_float(w[i] << 16) - mu, a1 = __uint_as_float(w[i] & 0xFFFF0000u) - mu;
-      w[i] = f2bf2(a0, a1);
-      x[2 * i] = __uint_as_float(w[i] << 16);
-      x[2 * i + 1] = __uint_as_float(w[i] & 0xFFFF0000u);
-    }
-    v = ku4{w[0], w[1], w[2], w[3]};
-  } else {
-    unpack8(v, x);
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i) q[i] = EPS == 1 ? __fmaf_rn(x[i], x[i], e1) : EPS == 2 ? x[i] * x[i] + e1 : x[i] * x[i];
-}
-// q of a chunk whose values are final (GC'd in place by sq_chunk).
-template <int EPS>
-__device__ __forceinline__ void sq_plain(const ku4 v, float e1, float q[8]) {
-  float x[8];
-  unpack8(v, x);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) q[i] = EPS == 1 ? __fmaf_rn(x[i], x[i], e1) : EPS == 2 ? x[i] * x[i] + e1 : x[i] * x[i];
-}
-
-// Column partial of a slice, segment by segment: segment k is chunk k of
-// every lane (columns 512k .. 512k+511).  Each wave writes its wave group's
-// partial for the segment into its LDS slot, and after one barrier every
-// thread forms the ordered sum ((w0 + w1) + w2) + w3 of two columns and
-// stores it (two LDS buffers alternate, so one barrier per segment suffices).
-__device__ __forceinline__ void seg_put(float (*seg)[512], int w, int lane, const float v[8]) {
-  kf4* d = (kf4*)(&seg[w][lane * 8]);
-  d[0] = kf4{v[0], v[1], v[2], v[3]};
-  d[1] = kf4{v[4], v[5], v[6], v[7]};
-}
-// The run partial (the slice partials added in slice order) is kept in
-// `racc` (LDS, C floats; each thread owns its two columns) and stored to
-// `part` after the last slice, or, with racc == nullptr, accumulated in
-// `part` itself.
-__device__ __forceinline__ void seg_fold(float (*seg)[512], int nw, int64_t col0, int64_t C, KAON_G float* part,
-                                         bool acc, bool last, int tid, float* racc) {
-  const int c = 2 * tid;
-  if (col0 + c >= C) return;  // C % 8 == 0: both columns are in range or neither
-  float a0 = seg[0][c], a1 = seg[0][c + 1];
-  for (int w = 1; w < nw; ++w) {
-    a0 = a0 + seg[w][c];
-    a1 = a1 + seg[w][c + 1];
-  }
-  KAON_G ku2* dst = (KAON_G ku2*)(part + col0 + c);
-  if (racc) {
-    float* r = racc + col0 + c;
-    if (acc) {
-      a0 = r[0] + a0;
-      a1 = r[1] + a1;
-    }
-    if (!last) {
-      r[0] = a0;
-      r[1] = a1;
-      return;
-    }
-  } else if (acc) {
-    const ku2 o = *dst;
-    a0 = __uint_as_float(o.x) + a0;
-    a1 = __uint_as_float(o.y) + a1;
-  }
-  *dst = ku2{__float_as_uint(a0), __float_as_uint(a1)};
-}
-// seg_fold with the run partial of the thread's two columns of segment k in
-// registers (r0, r1) instead of LDS; the order is the same.
-__device__ __forceinline__ void seg_fold_reg(float (*seg)[512], int nw, int64_t col0, int64_t C,
-                                             KAON_G float* part, bool acc, bool last, int tid, float& r0,
-                                             float& r1) {
-  const int c = 2 * tid;
-  if (col0 + c >= C) return;
-  float a0 = seg[0][c], a1 = seg[0][c + 1];
-  for (int w = 1; w < nw; ++w) {
-    a0 = a0 + seg[w][c];
-    a1 = a1 + seg[w][c + 1];
-  }
-  if (acc) {
-    a0 = r0 + a0;
-    a1 = r1 + a1;
-  }
-  if (!last) {
-    r0 = a0;
-    r1 = a1;
-    return;
-  }
-  *(KAON_G ku2*)(part + col0 + c) = ku2{__float_as_uint(a0), __float_as_uint(a1)};
-}
-
-// The second (clip) partial's run accumulator: racc2 in LDS (REG2 false), or
-// the thread's two columns per segment in registers rr2 (REG2 true).
-template <int CPL, int RW, int EPS, bool REG2>
-__device__ __forceinline__ void pf_stats_body(const KaonTensor& T, const KaonItem& it, const Ws& ws,
-                                              const KaonHyper& hp, int mode, float (*seg)[4][512],
-                                              KAON_G float* part, bool acc, bool last, float* racc,
-                                              KAON_G float* part2, float* racc2, float (&rr2)[48]) {
-  const int64_t C = T.C;
-  const int nch = (int)(C >> 3);
-  WaveRows wr = wave_rows(it);
-  // recomputed per slice: values derived from the lane are not kept live
-  // across the slice loop
-  asm volatile("" : "+v"(wr.lane));
-  int tid = (int)threadIdx.x;
-  asm volatile("" : "+v"(tid));
-  const int nrows = (int)(wr.re - wr.rb);
-  const bool gc = (hp.flags & KAON_F_GC) != 0;
-  const float e1 = hp.eps1;
-  if (mode == 1 && (!gc || nrows <= 0)) return;
-  const int64_t rl = lane_row(wr.rb, nrows, wr.lane);
-  const float row_old = (mode == 0 && nrows > 0) ? G(T.row)[rl] : 0.0f;
-  const void* gsrc = ws.src(T, hp.flags);
-  ku4 raw[RW][CPL];
-  load_group<CPL, RW>((const uint16_t*)gsrc, wr.rb, nrows, it.row0, C, nch, wr.lane, raw);
-  // GC means of the wave's rows; both per-row divisions by C are exact
-  // through the fp64 reciprocal (div_r64)
-  const double rc = rcp64((float)C);
-  float mu[RW];
-  KAON_G float* mu_arr = ws.mu(T);
-#pragma unroll
-  for (int j = 0; j < RW; ++j) {
-    mu[j] = 0.0f;
-    if (j >= nrows || !gc) continue;
-    float a = 0.0f;
-#pragma unroll
-    for (int k = 0; k < CPL; ++k) {
-      if (wr.lane + 64 * k < nch) {
-        float x[8];
-        unpack8(raw[j][k], x);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) a = a + x[i];
-      }
-    }
-    mu[j] = rbf(div_r64(wave_csum(a), rc));
-    if (wr.lane == 0) mu_arr[wr.rb + j] = mu[j];
-  }
-  if (mode == 1) return;
-  // q = (G - mu)^2 (+eps1) once per element: into the row sums (lane order:
-  // chunk by chunk) and the wave group's column partial (row order)
-  const int nw = (int)min<int64_t>(4, ((int64_t)it.nrows + RW - 1) / RW);
-  // Segments per barrier: the wide class (REG2: the clip's run partial in
-  // registers) has the LDS for two, so it waits half as often.  The buffer
-  // sets alternate from one barrier group to the next, across both passes;
-  // each column's partials are added in the same order either way.
-  constexpr int SEGG = REG2 ? 2 : 1;
-  constexpr int NG = (CPL + SEGG - 1) / SEGG;  // barrier groups per pass
-  auto sbuf = [&](int pass, int k) { return seg[((pass * NG + k / SEGG) & 1) * SEGG + k % SEGG]; };
-  float a2[RW];
-#pragma unroll
-  for (int j = 0; j < RW; ++j) a2[j] = 0.0f;
-#pragma unroll
-  for (int k = 0; k < CPL; ++k) {
-    if (nrows > 0) {
-      float v[8];
-      const bool in = wr.lane + 64 * k < nch;
-#pragma unroll
-      for (int j = 0; j < RW; ++j) {
-        if (j < nrows) {
-          float q[8];
-          sq_chunk<EPS>(raw[j][k], mu[j], gc, e1, q);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            if (in) a2[j] = a2[j] + q[i];
-            v[i] = j == 0 ? q[i] : v[i] + q[i];
-          }
-        }
-      }
-      seg_put(sbuf(0, k), wr.w, wr.lane, v);
-    }
-    if (k % SEGG == SEGG - 1 || k == CPL - 1) {
-      __syncthreads();
-#pragma unroll
-      for (int kk = k - k % SEGG; kk <= k; ++kk)
-        seg_fold(sbuf(0, kk), nw, (int64_t)kk * 512, C, part, acc, last, tid, racc);
-    }
-  }
-  float wr_inv[RW];  // 1 / row_j (the new row) for the clip partial
-#pragma unroll
-  for (int j = 0; j < RW; ++j) {
-    wr_inv[j] = 0.0f;
-    if (j >= nrows) continue;
-    const float s2 = wave_csum(a2[j]);
-    const float rv = lane_val(row_old, j);
-    const float nr = klerp(rv, div_r64(s2, rc), hp.w2);
-    if (wr.lane == 0) G(T.row)[wr.rb + j] = nr;
-    wr_inv[j] = 1.0f / nr;
-  }
-  if (!clip_alg(hp, mode)) return;
-  // The clip's second column partial, t = (G * G) / row (no eps1: rows of
-  // zeros add nothing), from the registers (GC'd in place by the first pass),
-  // in the same wave-group / slice / run order.  The LDS segment buffers keep
-  // alternating from the first pass's.
-#pragma unroll
-  for (int k = 0; k < CPL; ++k) {
-    if (nrows > 0) {
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < RW; ++j) {
-        if (j < nrows) {
-          float q[8];
-          sq_plain<0>(raw[j][k], e1, q);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const float t = q[i] * wr_inv[j];
-            v[i] = j == 0 ? t : v[i] + t;
-          }
-        }
-      }
-      seg_put(sbuf(1, k), wr.w, wr.lane, v);
-    }
-    if (k % SEGG == SEGG - 1 || k == CPL - 1) {
-      __syncthreads();
-#pragma unroll
-      for (int kk = k - k % SEGG; kk <= k; ++kk) {
-        if (REG2)
-          seg_fold_reg(sbuf(1, kk), nw, (int64_t)kk * 512, C, part2, acc, last, tid, rr2[2 * kk], rr2[2 * kk + 1]);
-        else
-          seg_fold(sbuf(1, kk), nw, (int64_t)kk * 512, C, part2, acc, last, tid, racc2);
-      }
-    }
-  }
-}
-
-// Row class 0: 1-4 chunks per lane, 1 class 1: 5-10, class 2: 11-24; the
-// body is specialized on the exact chunks per lane and its rows per wave
-// group (RW = max(1, KAON_ROW_BUDGET / CPL)).
-#define KAON_COMMA ,
-#define KAON_PF_SWITCH(CLS, BODY, X, ...)                                                      \
-  switch (cpl) {                                                                                \
-    case 1: if (CLS == 0) BODY<1, 20 X>(__VA_ARGS__); break;                                   \
-    case 2: if (CLS == 0) BODY<2, 10 X>(__VA_ARGS__); break;                                   \
-    case 3: if (CLS == 0) BODY<3, 6 X>(__VA_ARGS__); break;                                    \
-    case 4: if (CLS == 0) BODY<4, 5 X>(__VA_ARGS__); break;                                    \
-    case 5: if (CLS == 1) BODY<5, 4 X>(__VA_ARGS__); break;                                    \
-    case 6: if (CLS == 1) BODY<6, 3 X>(__VA_ARGS__); break;                                    \
-    case 7: if (CLS == 1) BODY<7, 2 X>(__VA_ARGS__); break;                                    \
-    case 8: if (CLS == 1) BODY<8, 2 X>(__VA_ARGS__); break;                                    \
-    case 9: if (CLS == 1) BODY<9, 2 X>(__VA_ARGS__); break;                                    \
-    case 10: if (CLS == 1) BODY<10, 2 X>(__VA_ARGS__); break;                                  \
-    case 11: if (CLS == 2) BODY<11, 1 X>(__VA_ARGS__); break;                                  \
-    case 12: if (CLS == 2) BODY<12, 1 X>(__VA_ARGS__); break;                                  \
-    case 13: if (CLS == 2) BODY<13, 1 X>(__VA_ARGS__); break;                                  \
-    case 14: if (CLS == 2) BODY<14, 1 X>(__VA_ARGS__); break;                                  \
-    case 15: if (CLS == 2) BODY<15, 1 X>(__VA_ARGS__); break;                                  \
-    case 16: if (CLS == 2) BODY<16, 1 X>(__VA_ARGS__); break;                                  \
-    case 17: if (CLS == 2) BODY<17, 1 X>(__VA_ARGS__); break;                                  \
-    case 18: if (CLS == 2) BODY<18, 1 X>(__VA_ARGS__); break;                                  \
-    case 19: if (CLS == 2) BODY<19, 1 X>(__VA_ARGS__); break;                                  \
-    case 20: if (CLS == 2) BODY<20, 1 X>(__VA_ARGS__); break;                                  \
-    case 21: if (CLS == 2) BODY<21, 1 X>(__VA_ARGS__); break;                                  \
-    case 22: if (CLS == 2) BODY<22, 1 X>(__VA_ARGS__); break;                                  \
-    case 23: if (CLS == 2) BODY<23, 1 X>(__VA_ARGS__); break;                                  \
-    case 24: if (CLS == 2) BODY<24, 1 X>(__VA_ARGS__); break;                                  \
-  }
-
-template <int CLS, int EPS, bool REG2>
-__device__ __forceinline__ void pf_stats_run(const KaonTensor* __restrict__ D, const KaonItem* __restrict__ items,
-                                             const Ws& ws, const KaonHyper& hp, int mode, float (*seg)[4][512],
-                                             float* racc, float* racc2) {
-  const KaonItem it = items[blockIdx.x];
-  const KaonTensor& T = D[it.tensor];
-  // KProdigy's per-element v and its block-factored tensors: their own pass 1 kernels
-  if (T.full_v || T.fb_r) return;
-  zero_accumulators(T, it, ws, hp.codec);
-  const int cpl = (int)(((T.C >> 3) + 63) >> 6);
-  KAON_G float* part = run_part(ws, T, it);
-  KAON_G float* part2 = part + (int64_t)T.ngroups * T.C;
-  const int nsl = run_slices(it);
-  float rr2[48];
-#pragma unroll
-  for (int i = 0; i < 48; ++i) rr2[i] = 0.0f;
-#pragma clang loop unroll(disable)
-  for (int sl = 0; sl < nsl; ++sl) {
-    if (sl > 0) __syncthreads();  // the LDS fold buffers are reused
-    const KaonItem si = slice_item(it, sl);
-    KAON_PF_SWITCH(CLS, pf_stats_body, KAON_COMMA EPS KAON_COMMA REG2, T, si, ws, hp, mode, seg, part, sl > 0,
-                   sl + 1 == nsl, racc, part2, racc2, rr2)
-  }
-}
-
-// Classes 0 and 1 are held to 4 waves per SIMD (128 VGPRs).  Every class
-// keeps its run partial in LDS (rows of at most 2048, 5120 and 12288
-// elements) and stores it once per run.  The clip's second run partial is
-// kept in LDS too in class 0, accumulated in the workspace in class 1 (in
-// registers it would cost class 1 a wave per SIMD, measured slower) and kept
-// in registers in class 2, whose LDS already limits it to 2 waves per SIMD.
-template <int CLS, int EPS>
-__global__ __launch_bounds__(KAON_WG, 4) void k_pf_stats(const KaonTensor* __restrict__ D,
-                                                         const KaonItem* __restrict__ items, Ws ws, KaonHyper hp,
-                                                         int mode) {
-  __shared__ __attribute__((aligned(16))) float seg[2][4][512];
-  __shared__ __attribute__((aligned(16))) float racc[CLS == 0 ? 4 * 512 : 10 * 512];
-  __shared__ __attribute__((aligned(16))) float racc2[CLS == 0 ? 4 * 512 : 1];
-  pf_stats_run<CLS, EPS, false>(D, items, ws, hp, mode, seg, racc, CLS == 0 ? racc2 : nullptr);
-}
-template <int EPS>
-__global__ __launch_bounds__(KAON_WG) void k_pf_stats_wide(const KaonTensor* __restrict__ D,
-                                                           const KaonItem* __restrict__ items, Ws ws, KaonHyper hp,
-                                                           int mode) {
-  __shared__ __attribute__((aligned(16))) float seg[4][4][512];  // two buffer sets of two segments
-  __shared__ __attribute__((aligned(16))) float racc[24 * 512];
-  pf_stats_run<2, EPS, true>(D, items, ws, hp, mode, seg, racc, nullptr);
-}
-
-#undef KAON_PF_SWITCH
-#undef KAON_COMMA
 
 // =============================================================== phases 5/6
 // Momentum chunk load (raw codes / bits) and store.
@@ -2481,29 +1690,11 @@ int launch_elem(const KaonLaunch& L, Ws ws, const KaonHyper& h, int codec, hipSt
   return check_launch(PHASE == 5 ? "kaon: keep-count launch" : "kaon: apply launch");
 }
 
-using StatsFn = void (*)(const KaonTensor*, const KaonItem*, Ws, KaonHyper, int);
-// row classes (slices are sorted by class): 0-2 prefetching kernels, 3-5 rows
-// of <= 4, 10, 24 chunks per lane in registers, 6 streamed rows; dynamic LDS
-// holds one slice column partial
-constexpr int kClassMaxC[KAON_ROW_CLASSES] = {4 * 512, 10 * 512, 24 * 512, 4 * 512, 10 * 512, 24 * 512, kSeg};
-
-// eps: 0 none, 1 fused square (eps1 == 0 or >= 2^-100), 2 unfused (sq_chunk)
-template <int GT>
-StatsFn stats_fn_gt(int cls, int eps) {
-  switch (cls) {
-    case 0: return eps == 1 ? k_pf_stats<0, 1> : eps == 2 ? k_pf_stats<0, 2> : k_pf_stats<0, 0>;
-    case 1: return eps == 1 ? k_pf_stats<1, 1> : eps == 2 ? k_pf_stats<1, 2> : k_pf_stats<1, 0>;
-    case 2: return eps == 1 ? k_pf_stats_wide<1> : eps == 2 ? k_pf_stats_wide<2> : k_pf_stats_wide<0>;
-    case 3: return k_stats<GT, 4>;
-    case 4: return k_stats<GT, 10>;
-    case 5: return k_stats<GT, 24>;
-    case 6: return k_stats<GT, 0>;
-  }
-  return nullptr;
-}
-StatsFn stats_fn(int gt, int cls, int eps) {
-  if (gt == KAON_F16) return cls >= 3 && cls != 5 ? stats_fn_gt<KAON_F16>(cls, eps) : nullptr;
-  return gt == KAON_BF16 ? stats_fn_gt<KAON_BF16>(cls, eps) : stats_fn_gt<KAON_F32>(cls, eps);
+// Phase 1 (kaon_stats.hip), its failure as this unit's error text.
+int run_stats(const KaonLaunch& L, Ws ws, const KaonHyper& hp, int mode, hipStream_t st) {
+  const char* why = launch_stats(L, ws, hp, mode, st);
+  if (why) return fail(why);
+  return check_launch("kaon: row-statistics launch");
 }
 
 using MsamFn = void (*)(const KaonTensor*, const KaonItem*, KaonHyper, float, float, uint32_t, const float*);
@@ -2519,28 +1710,6 @@ MsamFn msam_fn(int pt, int codec) {
   else { KAON_MSAM_CASE(KAON_F32) }
 #undef KAON_MSAM_CASE
   return nullptr;
-}
-
-// Phase-1 launches, one per register class run (slices are sorted by class).
-// KProdigy's coupled decay reads p beside g: the prefetching classes 0-2 then
-// run on the register classes 3-5 of the same chunks per lane (the same order).
-int launch_stats(const KaonLaunch& L, Ws ws, const KaonHyper& hp, int mode, hipStream_t st) {
-  int32_t off = 0;
-  const bool generic = mode == 0 && (hp.flags & KAON_F_PD_COUPLED) != 0;
-  for (int cls = 0; cls < KAON_ROW_CLASSES; ++cls) {
-    const int32_t cnt = L.row_runs[cls];
-    if (cnt <= 0) continue;
-    if (cls < 3 && hp.g_dtype != KAON_BF16) return fail("kaon: prefetching row class planned for non-bf16 grads");
-    const int kcls = generic && cls < 3 ? cls + 3 : cls;
-    const int eps = !(hp.flags & KAON_F_EPS) ? 0 : (hp.eps1 == 0.0f || hp.eps1 >= 0x1p-100f) ? 1 : 2;
-    StatsFn fn = stats_fn(hp.g_dtype, kcls, eps);
-    if (!fn) return fail("kaon: no row-statistics kernel for this grad dtype and row class");
-    const size_t lds = (mode == 0 && kcls >= 3) ? sizeof(float) * (size_t)kClassMaxC[kcls] : 0;
-    hipLaunchKernelGGL(fn, dim3(cnt), dim3(KAON_WG), lds, st, L.descs, L.row_items + off, ws, hp, mode);
-    off += cnt;
-  }
-  if (off != L.n_row_items) return fail("kaon: slice class runs do not add up to n_row_items");
-  return check_launch("kaon: k_stats launch");
 }
 
 using MuonMomFn = void (*)(const KaonTensor*, const KaonItem*, Ws, KaonHyper);
@@ -2770,7 +1939,7 @@ int kaon_adakaon_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask,
     if (e) return fail("kaon: torch-order sum launch", (hipError_t)e);
   } else {
     if (mask & (1u << 1)) {
-      if ((rc = launch_stats(*L, ws, h, 0, st))) return rc;
+      if ((rc = run_stats(*L, ws, h, 0, st))) return rc;
     }
     if ((mask & (1u << 2)) && L->n_fin_items > 0) {
       hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, h);
@@ -2829,7 +1998,7 @@ int kaon_adamuon_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask,
   ho.g_dtype = KAON_BF16;
   ho.codec = KAON_MOM_NONE;
   if (mask & (1u << 1)) {
-    if ((rc = launch_stats(*L, ws, ho, 0, st))) return rc;
+    if ((rc = run_stats(*L, ws, ho, 0, st))) return rc;
   }
   if ((mask & (1u << 2)) && L->n_fin_items > 0) {
     hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, ho);
@@ -2871,7 +2040,7 @@ int kaon_adapnm_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask, 
   ElemFn f6 = flat_pnm6(h, h.codec);
   if (!f3 || !f5 || !f6) return fail("kaon_adapnm_step: unsupported dtype / codec combination");
   if (mask & (1u << 1)) {
-    if ((rc = launch_stats(*L, ws, h, 0, st))) return rc;
+    if ((rc = run_stats(*L, ws, h, 0, st))) return rc;
   }
   if ((mask & (1u << 2)) && L->n_fin_items > 0) {
     hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, h);
@@ -2975,7 +2144,7 @@ int kaon_kprodigy_pass1(const KaonLaunch* L, const KaonHyper* hp, void* stream) 
   hipLaunchKernelGGL(k_pd_zero, dim3(L->n_tensors), dim3(KAON_WG), 0, st, L->descs, ws, codec);
   if ((rc = check_launch("kaon: KProdigy zero launch"))) return rc;
   // the factored row/col EMAs (tensors with a per-element v return at once)
-  if ((rc = launch_stats(*L, ws, h, 0, st))) return rc;
+  if ((rc = run_stats(*L, ws, h, 0, st))) return rc;
   if (L->n_fin_items > 0) {
     hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, h);
     if ((rc = check_launch("kaon: k_fin launch"))) return rc;
@@ -3035,7 +2204,7 @@ int kaon_lion_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask, vo
     const int e = torch_phases(*L, ws, h, 1u << 1, 1, st);
     if (e) return fail("kaon: torch-order GC mean launch", (hipError_t)e);
   } else if (mask & (1u << 1)) {
-    if ((rc = launch_stats(*L, ws, h, 1, st))) return rc;
+    if ((rc = run_stats(*L, ws, h, 1, st))) return rc;
   }
   if ((mask & (1u << 5)) && ((h.flags & KAON_F_CAUTIOUS) || quant)) {
     if ((rc = launch_elem<KAON_OPT_LION, 5>(*L, ws, h, h.codec, st))) return rc;
