@@ -143,13 +143,28 @@ __device__ void zero_accumulators(const KaonTensor& T, const KaonItem& it, const
 
 // The clip's algebraic sum of squares (Adakaon, AdaMuon): the scalar words of
 // a tensor hold rm at 4 and the partial sums S_k at 5 + k (one per finalize
-// item of KAON_COLITEM columns, or one for a 1-D tensor); phase 4 forms
+// item of KAON_COLITEM columns, or one for a 1-D tensor); clip_div forms
 // ss = rm * (S_0 + S_1 + ...) in item order.
 __device__ __forceinline__ int clip_parts(const KaonTensor& T) {
   return T.factored ? (int)((T.C + KAON_COLITEM - 1) / KAON_COLITEM) : 1;
 }
 __device__ __forceinline__ bool clip_alg(const KaonHyper& hp, int mode) {
   return mode == 0 && hp.clip > 0.0f && !(hp.flags & KAON_F_PNM);
+}
+// The tensor's clip divisor max(RMS(U) / clip, 1), RMS(U) = sqrt(ss) / sqrt(n)
+// (_factored.py:84-89 via adakaon.py:1001-1003): formed from the item sums by
+// each workgroup of phases 5 and 6 (Adakaon, AdaMuon; at most a few words, where
+// a launch of its own cost 5 us of a step); AdaPNM's and the torch-order step's
+// clip passes leave it in scalar word 0.
+__device__ __forceinline__ float clip_div(const KaonTensor& T, const Ws& ws, const KaonHyper& hp) {
+  const KAON_G float* sc = ws.scal(T);
+  if (hp.flags & (KAON_F_PNM | KAON_F_TORCH_ORDER)) return sc[0];
+  if (!(hp.clip > 0.0f)) return 1.0f;
+  const int np = clip_parts(T);
+  float S = 0.0f;
+  for (int k = 0; k < np; ++k) S = S + sc[5 + k];
+  const float ss = sc[4] * S;
+  return fmaxf((sqrtf(ss) / T.sqrt_n) / hp.clip, 1.0f);
 }
 // Workgroup sum of one value per thread: the 64-lane xor butterfly per wave,
 // then the four wave sums in order (valid in thread 0).  Every thread calls it.

@@ -337,8 +337,8 @@ __global__ __launch_bounds__(KAON_WG, PHASE == 5 ? 4 : 3) void k_flat(const Kaon
       if (ABSMAX && INT8) smax[k] = 0u;
     }
   };
-  // clip divisor of the tensor (phase 4), the cautious rescale
-  const float fac = !LION ? ws.scal(T)[0] : 1.0f;
+  // clip divisor of the tensor, the cautious rescale
+  const float fac = !LION ? clip_div(T, ws, hp) : 1.0f;
   const double rfac = rcp64(fac);
   double rden = 1.0;
   if (PHASE == 6 && cautious) {

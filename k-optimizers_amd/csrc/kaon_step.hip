@@ -71,52 +71,137 @@ int check_launch(const char* what) {
 // colsum2_j / col_j (thread t adds columns t, t+256, ... in order, then
 // wg_sum4).  kind 1: rm = mean(row) (canonical sum), rf = 1/sqrt(row/rm)
 // (_factored.py:48-52, 76-82); rm is kept in the tensor's scalar word 4.
-__device__ __forceinline__ float run_sum(const KAON_G float* part, int ngroups, int64_t C, int64_t j) {
-  float cs = 0.0f;
-  int g = 0;
-  for (; g + 8 <= ngroups; g += 8) {
-    float v[8];
+//
+// The work is a chain of run partials per column (315 of them for an embedding of
+// 50257 rows of 768) that one workgroup adds in order, so it is bound by how many
+// loads are in flight: kind 0 loads the next batch of runs of all the thread's
+// columns (and of both partials) before it adds the current one; kind 1 has the
+// four waves load 8 rounds of rows into LDS at a time for the one wave that adds.
+// One load batch after the other took 160-180 us for that embedding's net (124 M
+// params), this 68 us; 405 matrices of a UNet (677 M) 75 -> 37 us.
+template <int NC>
+__device__ __forceinline__ float fin_cols(const KaonTensor& T, const KaonItem& it, const Ws& ws, const KaonHyper& hp,
+                                          bool alg) {
+  constexpr int U = NC == 1 ? 12 : NC == 2 ? 8 : NC == 3 ? 6 : NC <= 5 ? 4 : 2;  // runs per batch
+  const int64_t C = T.C;
+  const int ng = T.ngroups;
+  const float fR = (float)T.R;
+  const KAON_G float* part = ws.part(T);
+  // without the clip sum the second partial's loads read the first again (dropped)
+  const KAON_G float* part2 = alg ? ws.part2(T) : part;
+  KAON_G float* cf = ws.cf(T);
+  const int64_t jend = (int64_t)it.row0 + it.nrows;
+  int64_t j[NC];
+  float cs[NC], c2[NC], old[NC];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = part[(int64_t)(g + u) * C + j];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) cs = cs + v[u];
+  for (int c = 0; c < NC; ++c) {
+    // threads past the item's columns read its last one
+    j[c] = min((int64_t)it.row0 + (int)threadIdx.x + KAON_WG * c, jend - 1);
+    cs[c] = c2[c] = 0.0f;
+    old[c] = T.col[j[c]];
   }
-  for (; g < ngroups; ++g) cs = cs + part[(int64_t)g * C + j];
-  return cs;
+  struct Batch {
+    float a[U][NC], b[U][NC];
+  };
+  auto load = [&](Batch& v, int g) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t off = (int64_t)min(g + u, ng - 1) * C;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        v.a[u][c] = part[off + j[c]];
+        v.b[u][c] = part2[off + j[c]];
+      }
+    }
+  };
+  auto add = [&](const Batch& v, int g) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (g + u >= ng) break;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        cs[c] = cs[c] + v.a[u][c];
+        c2[c] = c2[c] + v.b[u][c];
+      }
+    }
+  };
+  if (ng <= 2) {  // short tensors: no batch to fill
+    for (int g = 0; g < ng; ++g) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        cs[c] = cs[c] + part[(int64_t)g * C + j[c]];
+        c2[c] = c2[c] + part2[(int64_t)g * C + j[c]];
+      }
+    }
+  } else {
+    Batch b0, b1;
+    load(b0, 0);
+    for (int g = 0; g < ng; g += 2 * U) {
+      load(b1, g + U);
+      add(b0, g);
+      load(b0, g + 2 * U);
+      add(b1, g + U);
+    }
+  }
+  float a = 0.0f;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    if ((int64_t)it.row0 + (int)threadIdx.x + KAON_WG * c >= jend) continue;
+    const float nc = klerp(old[c], cs[c] / fR, hp.w2);
+    T.col[j[c]] = nc;
+    put_cf(cf, C, j[c], 1.0f / sqrtf(nc));
+    if (alg) a = a + c2[c] / nc;
+  }
+  return a;
 }
-__global__ __launch_bounds__(KAON_WG) void k_fin(const KaonTensor* __restrict__ D,
+__global__ __launch_bounds__(KAON_WG, 4) void k_fin(const KaonTensor* __restrict__ D,
                                                  const KaonItem* __restrict__ items, Ws ws, KaonHyper hp) {
+  constexpr int kRounds = 8;  // rounds of 64 chunks of rows in LDS
+  __shared__ float rows[kRounds * 512];
   __shared__ float rm_s;
   __shared__ float red4[4];
   const KaonItem it = items[blockIdx.x];
   const KaonTensor& T = D[it.tensor];
-  const int64_t R = T.R, C = T.C;
+  const int64_t R = T.R;
   if (it.kind == 0) {
     const bool alg = clip_alg(hp, 0);
-    const KAON_G float* part = ws.part(T);
-    const KAON_G float* part2 = ws.part2(T);
-    KAON_G float* cf = ws.cf(T);
     float a = 0.0f;
-    for (int64_t j = it.row0 + threadIdx.x; j < (int64_t)it.row0 + it.nrows; j += KAON_WG) {
-      const float cs = run_sum(part, T.ngroups, C, j);
-      const float nc = klerp(T.col[j], cs / (float)R, hp.w2);
-      T.col[j] = nc;
-      put_cf(cf, C, j, 1.0f / sqrtf(nc));
-      if (alg) a = a + run_sum(part2, T.ngroups, C, j) / nc;
+    switch ((it.nrows + KAON_WG - 1) / KAON_WG) {
+      case 1: a = fin_cols<1>(T, it, ws, hp, alg); break;
+      case 2: a = fin_cols<2>(T, it, ws, hp, alg); break;
+      case 3: a = fin_cols<3>(T, it, ws, hp, alg); break;
+      case 4: a = fin_cols<4>(T, it, ws, hp, alg); break;
+      case 5: a = fin_cols<5>(T, it, ws, hp, alg); break;
+      case 6: a = fin_cols<6>(T, it, ws, hp, alg); break;
+      case 7: a = fin_cols<7>(T, it, ws, hp, alg); break;
+      case 8: a = fin_cols<8>(T, it, ws, hp, alg); break;
     }
     if (alg) {
       const float S = wg_sum4(a, red4);
       if (threadIdx.x == 0) ws.scal(T)[5 + it.row0 / KAON_COLITEM] = S;
     }
   } else {
-    if (threadIdx.x < 64) {
-      const int64_t nch = (R + 7) >> 3;
-      float a = 0.0f;
-      for (int64_t c = threadIdx.x; c < nch; c += 64)
-        for (int i = 0; i < 8; ++i) {
-          const int64_t j = c * 8 + i;
-          if (j < R) a = a + T.row[j];
+    const KAON_G float* row = G(T.row);
+    float a = 0.0f;
+    for (int64_t r0 = 0; r0 < R; r0 += kRounds * 512) {
+      const int nr = (int)min<int64_t>(kRounds * 512, R - r0);
+      if (r0 > 0) __syncthreads();  // the rows are written again
+#pragma unroll 16
+      for (int k = threadIdx.x; k < nr; k += KAON_WG) rows[k] = row[r0 + k];
+      __syncthreads();
+      if (threadIdx.x < 64) {
+        for (int e = 8 * (int)threadIdx.x; e < nr; e += 512) {
+          if (e + 8 <= nr) {
+            const kf4 v0 = *(const kf4*)(rows + e), v1 = *(const kf4*)(rows + e + 4);
+            a = a + v0.x; a = a + v0.y; a = a + v0.z; a = a + v0.w;
+            a = a + v1.x; a = a + v1.y; a = a + v1.z; a = a + v1.w;
+          } else {
+            for (int i = e; i < nr; ++i) a = a + rows[i];
+          }
         }
+      }
+    }
+    if (threadIdx.x < 64) {
       const float s = wave_csum(a);
       if (threadIdx.x == 0) {
         rm_s = s / (float)R;
@@ -124,18 +209,24 @@ __global__ __launch_bounds__(KAON_WG) void k_fin(const KaonTensor* __restrict__ 
       }
     }
     __syncthreads();
-    const float rm = rm_s;
+    const double rrm = rcp64(rm_s);  // exact quotients (div_r64)
     KAON_G float* rf = ws.rf(T);
-    for (int64_t i = threadIdx.x; i < R; i += KAON_WG) rf[i] = 1.0f / sqrtf(T.row[i] / rm);
+    for (int64_t i0 = threadIdx.x; i0 < R; i0 += 16 * KAON_WG) {
+      float v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = row[min(i0 + u * KAON_WG, R - 1)];
+#pragma unroll
+      for (int u = 0; u < 16; ++u)
+        if (i0 + u * KAON_WG < R) rf[i0 + u * KAON_WG] = 1.0f / sqrtf(div_r64(v[u], rrm));
+    }
   }
 }
 
 // =============================================================== phase 4
-// Clip divisor of every tensor: max(RMS(U) / clip, 1), RMS(U) = sqrt(ss) /
-// sqrt(n) (_factored.py:84-89 via adakaon.py:1001-1003).  Adakaon and AdaMuon
-// take ss in the algebraic form rm * (S_0 + S_1 + ...) (the item partials in
-// item order, from phases 1-2); AdaPNM as the canonical sum over the row sums
-// rs of U^2 of its phase 3.  One wave per tensor.
+// Clip divisor of AdaPNM's tensors: max(RMS(U) / clip, 1), RMS(U) = sqrt(ss) /
+// sqrt(n) (_factored.py:84-89 via adakaon.py:1001-1003), ss the canonical sum over
+// the row sums rs of U^2 of its phase 3.  One wave per tensor.  (Adakaon and
+// AdaMuon form the divisor from the item sums in phases 5 and 6, clip_div.)
 __global__ __launch_bounds__(KAON_WG) void k_clipdiv(const KaonTensor* __restrict__ D, int32_t n_tensors, Ws ws,
                                                      KaonHyper hp) {
   const int t = (int)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -144,26 +235,17 @@ __global__ __launch_bounds__(KAON_WG) void k_clipdiv(const KaonTensor* __restric
   if (T.n == 0) return;
   const int lane = threadIdx.x & 63;
   const int64_t R = T.R;
-  float ss;
-  if (clip_alg(hp, 0)) {
-    const KAON_G float* sc = ws.scal(T);
-    const int np = clip_parts(T);
-    float S = 0.0f;
-    for (int k = 0; k < np; ++k) S = S + sc[5 + k];
-    ss = sc[4] * S;
-  } else {
-    const KAON_G float* rs = ws.rs(T);
-    float a = 0.0f;
-    for (int64_t c = lane; c * 8 < R; c += 64) {
-      float v[8];
+  const KAON_G float* rs = ws.rs(T);
+  float a = 0.0f;
+  for (int64_t c = lane; c * 8 < R; c += 64) {
+    float v[8];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = rs[min(c * 8 + i, R - 1)];
+    for (int i = 0; i < 8; ++i) v[i] = rs[min(c * 8 + i, R - 1)];
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (c * 8 + i < R) a = a + v[i];
-    }
-    ss = wave_csum(a);
+    for (int i = 0; i < 8; ++i)
+      if (c * 8 + i < R) a = a + v[i];
   }
+  const float ss = wave_csum(a);
   // clip_threshold 0 (AdaPNM) leaves the update unclipped (adapnm.py:157-161)
   if (lane == 0) ws.scal(T)[0] = hp.clip > 0.0f ? fmaxf((sqrtf(ss) / T.sqrt_n) / hp.clip, 1.0f) : 1.0f;
 }
@@ -1945,12 +2027,8 @@ int kaon_adakaon_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask,
       hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, h);
       if ((rc = check_launch("kaon: k_fin launch"))) return rc;
     }
-    // phase 3 (the clip's sum of squares) is folded into phases 1 and 2
-    if (mask & (1u << 4)) {
-      hipLaunchKernelGGL(k_clipdiv, dim3((L->n_tensors + 3) / 4), dim3(KAON_WG), 0, st, L->descs, L->n_tensors, ws,
-                         h);
-      if ((rc = check_launch("kaon: k_clipdiv launch"))) return rc;
-    }
+    // phase 3 (the clip's sum of squares) is folded into phases 1 and 2, phase 4 (its
+    // divisor) into phases 5 and 6
   }
   return elem_phases(*L);
 }
@@ -2004,11 +2082,8 @@ int kaon_adamuon_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask,
     hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, ho);
     if ((rc = check_launch("kaon: k_fin launch"))) return rc;
   }
-  // phase 3 (the clip's sum of squares) is folded into phases 1 and 2
-  if (mask & (1u << 4)) {
-    hipLaunchKernelGGL(k_clipdiv, dim3((L->n_tensors + 3) / 4), dim3(KAON_WG), 0, st, L->descs, L->n_tensors, ws, ho);
-    if ((rc = check_launch("kaon: k_clipdiv launch"))) return rc;
-  }
+  // phase 3 (the clip's sum of squares) is folded into phases 1 and 2, phase 4 (its
+  // divisor) into phases 5 and 6
   // 5-6: cautious count against the grad; requant, write
   if ((mask & (1u << 5)) && (h.flags & KAON_F_CAUTIOUS)) {
     if ((rc = launch_elem<KAON_OPT_ADAMUON, 5>(*L, ws, h, codec, st))) return rc;
