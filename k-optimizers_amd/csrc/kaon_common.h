@@ -129,7 +129,10 @@ __device__ __forceinline__ int chunk_cnt(int64_t c, int64_t C) {
 // Zero what phase 5 accumulates with atomics (keep-count; int8 row absmax, 4-bit
 // block absmax).  Run by the phase-1 slice.
 __device__ void zero_accumulators(const KaonTensor& T, const KaonItem& it, const Ws& ws, int codec) {
-  if (it.row0 == 0 && threadIdx.x == 0) ((KAON_G uint32_t*)ws.scal(T))[1] = 0u;
+  if (it.row0 == 0 && threadIdx.x == 0) {
+    ((KAON_G uint32_t*)ws.scal(T))[1] = 0u;
+    ((KAON_G uint32_t*)ws.scal(T))[2] = 0x7F800000u;  // AdaPNM: KeepEarly's minimum
+  }
   if (codec == KAON_MOM_INT8) {
     for (int64_t r = it.row0 + threadIdx.x; r < (int64_t)it.row0 + it.nrows; r += KAON_WG) ws.ramax(T)[r] = 0u;
   } else if (codec == KAON_MOM_4BIT) {
@@ -166,6 +169,50 @@ __device__ __forceinline__ float clip_div(const KaonTensor& T, const Ws& ws, con
   const float ss = sc[4] * S;
   return fmaxf((sqrtf(ss) / T.sqrt_n) / hp.clip, 1.0f);
 }
+// AdaPNM's cautious keep count, taken in its clip-sum pass (phase 3) instead of a
+// pass of its own.  The count is of d * g > 0 with d = (u / fac) * lr, and fac is
+// known only after that pass; u * g > 0 gives the same bit wherever neither d nor
+// the product d * g underflows.  So phase 3 counts u * g > 0 and keeps the least
+// |u| and u * g of the counted elements in scalar word 2; with fac known, phase 4
+// (k_clipdiv) checks that minimum scaled by lr / fac against 2^-120 (far above the
+// rounding of d and d * g) and lr <= 1/2 (an uncounted product that underflowed
+// stays 0 when scaled down; fac >= 1).  A tensor that fails has its count cleared
+// and word 3 set, and only then does phase 5 count it.  NaN counts in neither form,
+// and a fac that is inf or NaN fails the check.  Two bf16 momenta, 677 M params:
+// the keep-count pass took 622 us (6 B/param read), its early exit takes 14 us and
+// the count adds 20 us to the clip-sum pass.
+struct KeepEarly {
+  uint32_t keep = 0;
+  float least = __builtin_inff();
+  __device__ __forceinline__ void add(float u, float g, bool in) {
+    const float x = u * g;
+    const bool k = x > 0.0f && in;
+    keep += k ? 1u : 0u;
+    least = fminf(least, k ? fminf(fabsf(u), x) : least);
+  }
+  // every thread of the workgroup calls it
+  __device__ __forceinline__ void flush(const KaonTensor& T, const Ws& ws) {
+    __shared__ uint32_t ks[4];
+    __shared__ uint32_t ls[4];
+    const uint32_t k = wave_sum_u32(keep);
+    const uint32_t l = wave_butterfly(__float_as_uint(least), [](uint32_t a, uint32_t b) { return a < b ? a : b; });
+    if ((threadIdx.x & 63) == 0) {
+      ks[threadIdx.x >> 6] = k;
+      ls[threadIdx.x >> 6] = l;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const uint32_t tot = ks[0] + ks[1] + ks[2] + ks[3];
+      if (tot) {
+        atomicAdd(ws.keep_ctr(T), tot);
+        atomicMin(ws.keep_ctr(T) + 1, min(min(ls[0], ls[1]), min(ls[2], ls[3])));
+      }
+    }
+  }
+};
+// Whether phase 5 still has to count this AdaPNM tensor.
+__device__ __forceinline__ bool keep_late(const KaonTensor& T, const Ws& ws) { return ws.keep_ctr(T)[2] != 0u; }
+
 // Workgroup sum of one value per thread: the 64-lane xor butterfly per wave,
 // then the four wave sums in order (valid in thread 0).  Every thread calls it.
 __device__ __forceinline__ float wg_sum4(float a, float* red) {

@@ -566,6 +566,7 @@ __global__ __launch_bounds__(KAON_WG) void k_fast(const KaonTensor* __restrict__
   __shared__ uint32_t keep_s[4];
   const KaonItem it = items[blockIdx.x];
   const KaonTensor& T = D[it.tensor];
+  if (PNM && PHASE == 5 && !keep_late(T, ws)) return;
   const uint32_t C = (uint32_t)T.C;
   const int64_t n = T.n;
   const uint32_t nfull = C >> 3;  // full chunks per row
@@ -803,8 +804,8 @@ ElemFn fast_by_flags(int ff) {
     case FF_GC | FF_CAUT: return k_fast<OPT, PHASE, CODEC, FF_GC | FF_CAUT>;
     case FF_GC | FF_CAUT | FF_WD: return k_fast<OPT, PHASE, CODEC, FF_GC | FF_CAUT | FF_WD>;
   }
-  if constexpr (PHASE == 6 && (OPT == KAON_OPT_ADAKAON || OPT == KAON_OPT_LION)) {
-    // Lion, and Adakaon off its fused path, leave p.grad centralized (the
+  if constexpr (PHASE == 6 && (OPT == KAON_OPT_ADAKAON || OPT == KAON_OPT_LION || OPT == KAON_OPT_ADAPNM)) {
+    // Lion, and Adakaon and AdaPNM off their fused paths, leave p.grad centralized (the
     // reference's native path)
     switch (ff) {
       case FF_GC | FF_CAUT | FF_GCW: return k_fast<OPT, PHASE, CODEC, FF_GC | FF_CAUT | FF_GCW>;

@@ -246,6 +246,7 @@ __global__ __launch_bounds__(KAON_WG, PHASE == 5 ? 4 : 3) void k_flat(const Kaon
   __shared__ uint32_t keep_s[4];
   const KaonItem it = items[blockIdx.x];
   const KaonTensor& T = D[it.tensor];
+  if (PNM && PHASE == 5 && !keep_late(T, ws)) return;
   const int64_t n = T.n;
   const uint32_t C = (uint32_t)T.C;
   const int lane = threadIdx.x & 63;
@@ -253,7 +254,7 @@ __global__ __launch_bounds__(KAON_WG, PHASE == 5 ? 4 : 3) void k_flat(const Kaon
   const bool factored = T.factored != 0;
   const bool gc = (hp.flags & KAON_F_GC) && factored;
   const bool gcw = PHASE == 6 && gc && (hp.flags & KAON_F_GC_WRITE) && T.gc_write &&
-                   (OPT == KAON_OPT_ADAKAON || LION);
+                   (OPT == KAON_OPT_ADAKAON || LION || PNM);
   const bool cautious = (hp.flags & KAON_F_CAUTIOUS) != 0;
   const bool wd = (hp.flags & KAON_F_WD) != 0;
   const bool nk_remove = OPT == KAON_OPT_ADAKAON && MOM && (hp.flags & KAON_F_NK_REMOVE);

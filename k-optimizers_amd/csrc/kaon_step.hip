@@ -246,8 +246,16 @@ __global__ __launch_bounds__(KAON_WG) void k_clipdiv(const KaonTensor* __restric
       if (c * 8 + i < R) a = a + v[i];
   }
   const float ss = wave_csum(a);
-  // clip_threshold 0 (AdaPNM) leaves the update unclipped (adapnm.py:157-161)
-  if (lane == 0) ws.scal(T)[0] = hp.clip > 0.0f ? fmaxf((sqrtf(ss) / T.sqrt_n) / hp.clip, 1.0f) : 1.0f;
+  // clip_threshold 0 leaves the update unclipped (adapnm.py:157-161)
+  if (lane == 0) {
+    const float fac = hp.clip > 0.0f ? fmaxf((sqrtf(ss) / T.sqrt_n) / hp.clip, 1.0f) : 1.0f;
+    KAON_G uint32_t* w = (KAON_G uint32_t*)ws.scal(T);
+    ws.scal(T)[0] = fac;
+    // whether phase 3's keep count holds (KeepEarly)
+    const bool ok = hp.lr <= 0.5f && __uint_as_float(w[2]) * (hp.lr / fac) >= 0x1p-120f;
+    w[3] = ok ? 0u : 1u;
+    if (!ok) w[1] = 0u;
+  }
 }
 
 // =============================================================== phases 5/6
@@ -520,9 +528,10 @@ __global__ __launch_bounds__(KAON_WG) void k_muon_norm(const KaonTensor* __restr
 //   u      = pn * ((r * c) * bc2)                   factored
 //          = pn / ((sqrt(v + 1e-15) + eps) / bc2)   1-D (max_v under ams_bound)
 //   d      = (u / fac) * lr / (1 - b1^t)
-// Phase 3 (slices of row runs): the row sums of u^2 for the clip, and the
-// absmax of m_pos' per int8 row / 4-bit block with the old scales.  Phase 5:
-// the cautious keep count of d * g > 0.  Phase 6: requantize or store m_pos',
+// Phase 3 (slices of row runs): the row sums of u^2 for the clip, the absmax of
+// m_pos' per int8 row / 4-bit block with the old scales, and the cautious keep
+// count of d * g > 0 (KeepEarly; phase 5 counts again only tensors whose count
+// could depend on the clip).  Phase 6: requantize or store m_pos',
 // write p after the decoupled decay p * (1 - lr*wd).  The negative buffer is
 // only read.  Odd steps take m as the positive buffer, even steps m2.
 template <int GT, int CODEC>
@@ -554,6 +563,7 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
   // the scales of the last 4-bit block visited: read once per run of its elements
   uint32_t c_blk = 0xFFFFFFFFu;
   float c_o = 1.0f, c_g = 1.0f;
+  KeepEarly ke;
 
   for (int64_t r = wr.rb; r < wr.re; ++r) {
     const float mu = gc ? uniform_f(ws.mu(T)[r]) : 0.0f;
@@ -635,6 +645,7 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
         const float pn = __fmaf_rn(hp.pn_neg, mng, mfv * hp.pn_pos) * hp.pn_rnorm;
         const float u = factored ? pn * ((rf * f[i]) * hp.bc2) : pn / ((sqrtf(f[i] + 1e-15f) + hp.eps1) / hp.bc2);
         ss = ss + u * u;
+        ke.add(u, g[i], true);
         if (QUANT) {
           const float ax = fabsf(mfv);
           if (CODEC == KAON_MOM_INT8) {
@@ -658,6 +669,7 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
     if (wr.lane == 0) ws.rs(T)[r] = s2;
   }
   if (CODEC == KAON_MOM_4BIT) bm4.flush(ws.bamax(T));
+  if (hp.flags & KAON_F_CAUTIOUS) ke.flush(T, ws);
 }
 
 // AdaPNM phase 3 on row class 0 (factored, bf16 g, 16-byte rows with
@@ -669,7 +681,7 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
 // chunks, so every load is unconditional.
 template <int CPL, int GR, int CODEC>
 __device__ __forceinline__ void pnm_ss_body(const KaonTensor& T, const KaonItem& it, const Ws& ws,
-                                            const KaonHyper& hp) {
+                                            const KaonHyper& hp, KeepEarly& ke) {
   constexpr bool I8 = CODEC == KAON_MOM_INT8;
   const uint32_t C = (uint32_t)T.C;
   const int nch = (int)(C >> 3);
@@ -759,6 +771,7 @@ __device__ __forceinline__ void pnm_ss_body(const KaonTensor& T, const KaonItem&
           const float pn = __fmaf_rn(hp.pn_neg, mn[i], mfv * hp.pn_pos) * hp.pn_rnorm;
           const float u = pn * ((rf * f[i]) * hp.bc2);
           ss = ss + u * u;
+          ke.add(u, g[i], true);
           if (I8) amax = fmaxf(amax, fabsf(mfv));
         }
       }
@@ -787,15 +800,17 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm_ss(const KaonTensor* __restrict
   const KaonTensor& T = D[it.tensor];
   const int cpl = (int)(((T.C >> 3) + 63) >> 6);
   constexpr int W = CODEC == KAON_MOM_INT8 ? 10 : 6;  // rows x chunks held per group
+  KeepEarly ke;
 #define KAON_PNM_SS(N)                                                                 \
   case N: {                                                                            \
     constexpr int GR = W / N > 0 ? W / N : 1;                                          \
-    pnm_ss_body<N, GR, CODEC>(T, it, ws, hp);                                          \
+    pnm_ss_body<N, GR, CODEC>(T, it, ws, hp, ke);                                      \
     break;                                                                             \
   }
   switch (cpl) {
     KAON_PNM_SS(1) KAON_PNM_SS(2) KAON_PNM_SS(3) KAON_PNM_SS(4)
   }
+  if (hp.flags & KAON_F_CAUTIOUS) ke.flush(T, ws);
 #undef KAON_PNM_SS
 }
 

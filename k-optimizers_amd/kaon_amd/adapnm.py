@@ -166,6 +166,8 @@ class AdaPNM(KaonOptimizer):
         flags = L.F_MOMENTUM
         if group["gradient_centralization"]:
             flags |= L.F_GC
+            if self.centralize_grads_in_place:
+                flags |= L.F_GC_WRITE  # the apply stores the centralized gradient
         if group["cautious"]:
             flags |= L.F_CAUTIOUS
         if wd != 0:
@@ -197,7 +199,6 @@ class AdaPNM(KaonOptimizer):
                 hp = self._hyper(group, pdt, gdt)
                 L.check(lib.kaon_adapnm_step(ctypes.byref(plan.launch), ctypes.byref(hp), E.stream_handle(dev)),
                         "kaon_adapnm_step")
-                self._gc_writeback(group, plan, hp, dev)
         return loss
 
     def _build_launches(self, gid: int, group: dict[str, Any], params: list[torch.Tensor],
