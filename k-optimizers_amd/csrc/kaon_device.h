@@ -30,6 +30,12 @@ __device__ __forceinline__ KAON_G T* G(T* p) {
 typedef uint32_t ku4 __attribute__((ext_vector_type(4)));
 typedef uint32_t ku2 __attribute__((ext_vector_type(2)));
 typedef float kf4 __attribute__((ext_vector_type(4)));
+// the same at any address: gfx950 loads and stores 16 bytes unaligned with the
+// same instructions, so a chunk of 8 elements needs no alignment of its own
+typedef ku4 ku4_any __attribute__((aligned(1)));
+typedef ku2 ku2_any __attribute__((aligned(1)));
+typedef kf4 kf4_any __attribute__((aligned(4)));
+typedef uint32_t ku1_any __attribute__((aligned(1)));
 
 // ------------------------------------------------------------------ bf16
 __device__ __forceinline__ float bf2f(uint32_t h) { return __uint_as_float(h << 16); }
@@ -153,15 +159,30 @@ __device__ __forceinline__ void noise8(uint64_t seed, uint32_t step, uint32_t ti
   }
 }
 
-// Noise word of one element (any alignment).
-__device__ __forceinline__ uint32_t noise1(uint64_t seed, uint32_t step, uint32_t tid, uint32_t stream,
-                                           int64_t e, const uint16_t* inj) {
-  if (inj) return G(inj)[e];
-  const uint64_t ch = (uint64_t)e >> 3;
-  uint32_t c[4] = {(uint32_t)ch, (uint32_t)(ch >> 32), tid, stream};
-  philox10(c, (uint32_t)seed, step);
-  const int wi = (int)(e & 7);
-  return (c[wi >> 1] >> ((wi & 1) * 16)) & 0xFFFFu;
+// noise8 of the eight elements from any e0: they lie in two aligned chunks, whose
+// words are shifted down by e0 % 8.
+__device__ __forceinline__ void noise8_any(uint64_t seed, uint32_t step, uint32_t tid, uint32_t stream, int64_t e0,
+                                           const uint16_t* inj, int cnt, uint32_t w[8]) {
+  const uint32_t s = (uint32_t)e0 & 7u;
+  if (inj || s == 0u) {
+    noise8(seed, step, tid, stream, e0, inj, cnt, w);
+    return;
+  }
+  const uint64_t ch = (uint64_t)e0 >> 3;
+  uint32_t r[8] = {(uint32_t)ch, (uint32_t)(ch >> 32), tid, stream,
+                   (uint32_t)(ch + 1), (uint32_t)((ch + 1) >> 32), tid, stream};
+  philox10(r, (uint32_t)seed, step);
+  philox10(r + 4, (uint32_t)seed, step);
+#pragma unroll
+  for (int k = 0; k < 6; ++k) r[k] = (s & 4u) ? r[k + 2] : r[k];
+#pragma unroll
+  for (int k = 0; k < 5; ++k) r[k] = (s & 2u) ? r[k + 1] : r[k];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const uint32_t v = (s & 1u) ? (r[k] >> 16) | (r[k + 1] << 16) : r[k];
+    w[2 * k] = v & 0xFFFFu;
+    w[2 * k + 1] = v >> 16;
+  }
 }
 
 // _add_stochastic_bf16_ bit trick: int32 add of the 16-bit noise, clear the
@@ -181,13 +202,14 @@ __device__ __forceinline__ uint32_t pack_hi16(uint32_t lo, uint32_t hi) {
 }
 
 // ------------------------------------------------------------------ loads
-// Chunk loads into fp32 (8 elements, `cnt` valid; vec = 16-byte vector path).
+// Chunk loads into fp32 (8 elements, `cnt` valid; vec = 16-byte vector path, which
+// reads all 8 whatever cnt is, at any alignment).
 template <int DT>
 __device__ __forceinline__ void ld8(const void* base, int64_t off, int cnt, bool vec, float o[8]) {
   if (DT == KAON_BF16) {
     const KAON_G uint16_t* b = G((const uint16_t*)base + off);
     if (vec) {
-      const ku4 v = *(const KAON_G ku4*)b;
+      const ku4 v = *(const KAON_G ku4_any*)b;
       const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -201,7 +223,7 @@ __device__ __forceinline__ void ld8(const void* base, int64_t off, int cnt, bool
   } else if (DT == KAON_F16) {
     const KAON_G uint16_t* b = G((const uint16_t*)base + off);
     if (vec) {
-      const ku4 v = *(const KAON_G ku4*)b;
+      const ku4 v = *(const KAON_G ku4_any*)b;
       const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -215,8 +237,8 @@ __device__ __forceinline__ void ld8(const void* base, int64_t off, int cnt, bool
   } else {
     const KAON_G float* b = G((const float*)base + off);
     if (vec) {
-      const kf4 v0 = *(const KAON_G kf4*)b;
-      const kf4 v1 = *(const KAON_G kf4*)(b + 4);
+      const kf4 v0 = *(const KAON_G kf4_any*)b;
+      const kf4 v1 = *(const KAON_G kf4_any*)(b + 4);
       o[0] = v0.x; o[1] = v0.y; o[2] = v0.z; o[3] = v0.w;
       o[4] = v1.x; o[5] = v1.y; o[6] = v1.z; o[7] = v1.w;
     } else {
@@ -230,7 +252,7 @@ __device__ __forceinline__ void ld8(const void* base, int64_t off, int cnt, bool
 __device__ __forceinline__ void ld8_bits(const void* base, int64_t off, int cnt, bool vec, uint32_t o[8]) {
   const KAON_G uint16_t* b = G((const uint16_t*)base + off);
   if (vec) {
-    const ku4 v = *(const KAON_G ku4*)b;
+    const ku4 v = *(const KAON_G ku4_any*)b;
     const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -250,7 +272,7 @@ __device__ __forceinline__ void st8_bits(void* base, int64_t off, int cnt, bool 
     v.y = (o[2] & 0xFFFFu) | (o[3] << 16);
     v.z = (o[4] & 0xFFFFu) | (o[5] << 16);
     v.w = (o[6] & 0xFFFFu) | (o[7] << 16);
-    *(KAON_G ku4*)b = v;
+    *(KAON_G ku4_any*)b = v;
   } else {
 #pragma unroll
     for (int i = 0; i < 8; ++i)
@@ -260,8 +282,8 @@ __device__ __forceinline__ void st8_bits(void* base, int64_t off, int cnt, bool 
 __device__ __forceinline__ void st8_f32(void* base, int64_t off, int cnt, bool vec, const float o[8]) {
   KAON_G float* b = G((float*)base + off);
   if (vec) {
-    *(KAON_G kf4*)b = kf4{o[0], o[1], o[2], o[3]};
-    *(KAON_G kf4*)(b + 4) = kf4{o[4], o[5], o[6], o[7]};
+    *(KAON_G kf4_any*)b = kf4{o[0], o[1], o[2], o[3]};
+    *(KAON_G kf4_any*)(b + 4) = kf4{o[4], o[5], o[6], o[7]};
   } else {
 #pragma unroll
     for (int i = 0; i < 8; ++i)

@@ -265,7 +265,7 @@ __device__ __forceinline__ void ld_mom_at(const void* mbuf, int64_t e0, int cnt,
   if (CODEC == KAON_MOM_INT8) {
     const int8_t* m = (const int8_t*)mbuf + e0;
     if (vec) {
-      const ku2 v = *(const KAON_G ku2*)G(m);
+      const ku2 v = *(const KAON_G ku2_any*)G(m);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         q[i] = (v.x >> (8 * i)) & 0xFFu;
@@ -311,7 +311,7 @@ __device__ __forceinline__ void st_mom_at(void* mbuf, int64_t n, int64_t e0, int
       ku2 v;
       v.x = (q[0] & 0xFF) | ((q[1] & 0xFF) << 8) | ((q[2] & 0xFF) << 16) | ((q[3] & 0xFF) << 24);
       v.y = (q[4] & 0xFF) | ((q[5] & 0xFF) << 8) | ((q[6] & 0xFF) << 16) | ((q[7] & 0xFF) << 24);
-      *(KAON_G ku2*)G(m) = v;
+      *(KAON_G ku2_any*)G(m) = v;
     } else {
 #pragma unroll
       for (int i = 0; i < 8; ++i)
@@ -323,7 +323,7 @@ __device__ __forceinline__ void st_mom_at(void* mbuf, int64_t n, int64_t e0, int
       uint32_t v = 0;
 #pragma unroll
       for (int i = 0; i < 8; ++i) v |= (q[i] & 0xFu) << (4 * i);
-      *(uint32_t*)(m + (e0 >> 1)) = v;
+      *(KAON_G ku1_any*)G(m + (e0 >> 1)) = v;
     } else {
       // bytes shared with a neighbouring chunk (odd starts) are merged with an
       // atomic; the byte of an odd-length tensor's last element keeps 0 in its
@@ -408,7 +408,6 @@ __global__ __launch_bounds__(KAON_WG) void k_muon_mom(const KaonTensor* __restri
   const int64_t C = T.C;
   const int64_t nch = (C + 7) >> 3;
   const int cpl = (int)((nch + 63) >> 6);
-  const bool vec = T.vec_rows != 0;
   const bool gc = (hp.flags & KAON_F_GC) != 0;
   const bool mom = (hp.flags & KAON_F_MOMENTUM) != 0 && CODEC != KAON_MOM_NONE;
   const int64_t B = CODEC == KAON_MOM_4BIT ? (int64_t)T.block4 : 1;
@@ -427,7 +426,7 @@ __global__ __launch_bounds__(KAON_WG) void k_muon_mom(const KaonTensor* __restri
         const int cnt = chunk_cnt(c, C);
         if (cnt <= 0) continue;
         float x[8];
-        ld8<GT>(T.g, r * C + c * 8, cnt, vec && cnt == 8, x);
+        ld8<GT>(T.g, r * C + c * 8, cnt, r * C + c * 8 + 8 <= T.n, x);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
           if (i < cnt) a = a + x[i];
@@ -443,15 +442,16 @@ __global__ __launch_bounds__(KAON_WG) void k_muon_mom(const KaonTensor* __restri
       const int cnt = chunk_cnt(c, C);
       if (cnt <= 0) continue;
       const int64_t e0 = r * C + c * 8;
-      const bool vv = vec && cnt == 8;
+      // a row's partial last chunk reads on into the next row (not past the tensor)
+      const bool vv = cnt == 8, vl = e0 + 8 <= T.n;
       float g[8];
-      ld8<GT>(T.g, e0, cnt, vv, g);
+      ld8<GT>(T.g, e0, cnt, vl, g);
       if (gc) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) g[i] = round_to<GT>(g[i] - mu);
       }
       uint32_t mq[8];
-      if (mom) ld_mom_raw<CODEC>(T, e0, cnt, vv, mq);
+      if (mom) ld_mom_raw<CODEC>(T, e0, cnt, vl, mq);
       uint32_t qout[8], mob[8];
       float Mv[8];
 #pragma unroll
@@ -485,7 +485,7 @@ __global__ __launch_bounds__(KAON_WG) void k_muon_mom(const KaonTensor* __restri
         mob[i] = xb;
       }
       if (vv) {
-        *(KAON_G ku4*)(mo + e0) = ku4{mob[0] | (mob[1] << 16), mob[2] | (mob[3] << 16), mob[4] | (mob[5] << 16),
+        *(KAON_G ku4_any*)(mo + e0) = ku4{mob[0] | (mob[1] << 16), mob[2] | (mob[3] << 16), mob[4] | (mob[5] << 16),
                                       mob[6] | (mob[7] << 16)};
       } else {
         for (int i = 0; i < cnt; ++i) mo[e0 + i] = (uint16_t)mob[i];
@@ -545,7 +545,6 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
   const int64_t C = T.C;
   const int64_t nch = (C + 7) >> 3;
   const int cpl = (int)((nch + 63) >> 6);
-  const bool vec_t = T.vec_rows != 0;
   const bool factored = T.factored != 0;
   const bool gc = (hp.flags & KAON_F_GC) && factored;
   const bool ams = (hp.flags & KAON_F_AMS) && !factored && T.max_v;
@@ -585,13 +584,15 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
       if (cnt <= 0) continue;
       const int64_t j0 = c * 8;
       const int64_t e0 = r * C + j0;
-      const bool vec = vec_t && cnt == 8;
+      // a row's partial last chunk reads on into the next row (not past the tensor;
+      // the column factors have 8 words beyond C)
+      const bool vec = e0 + 8 <= T.n;
       float g[8], f[8];
       uint32_t mq[8], nq[8];
       ld8<GT>(T.g, e0, cnt, vec, g);
       ld_mom_at<CODEC>(mpos, e0, cnt, vec, mq);
       ld_mom_at<CODEC>(mneg, e0, cnt, vec, nq);
-      ld8<KAON_F32>(fsrc, j0, cnt, vec, f);
+      ld8<KAON_F32>(fsrc, j0, cnt, vec || factored, f);
       if (gc) {
 #pragma unroll
         for (int i = 0; i < 8; i += 2) {
@@ -829,7 +830,6 @@ __global__ __launch_bounds__(KAON_WG) void k_msq(const KaonTensor* __restrict__ 
   const int64_t C = T.C;
   const int64_t nch = (C + 7) >> 3;
   const int cpl = (int)((nch + 63) >> 6);
-  const bool vec = T.vec_rows != 0;
   const WaveRows wr = wave_rows(it);
   for (int64_t r = wr.rb; r < wr.re; ++r) {
     const float sc = CODEC == KAON_MOM_INT8 ? uniform_f(G(T.m_scale)[T.factored ? r : 0]) : 1.0f;
@@ -840,7 +840,7 @@ __global__ __launch_bounds__(KAON_WG) void k_msq(const KaonTensor* __restrict__ 
       if (cnt <= 0) continue;
       const int64_t e0 = r * C + c * 8;
       uint32_t mq[8];
-      ld_mom_at<CODEC>(T.m, e0, cnt, vec && cnt == 8, mq);
+      ld_mom_at<CODEC>(T.m, e0, cnt, e0 + 8 <= T.n, mq);
       // 4-bit: walk the blocks from the chunk's first element (32-bit: n < 2^32)
       uint32_t blk = 0u, boff = 0u;
       if (CODEC == KAON_MOM_4BIT) {
@@ -987,7 +987,6 @@ __global__ __launch_bounds__(KAON_WG) void k_pd1(const KaonTensor* __restrict__ 
   const int64_t C = T.C;
   const int64_t nch = (C + 7) >> 3;
   const int cpl = (int)((nch + 63) >> 6);
-  const bool vec = T.vec_rows != 0;
   const bool gc = (hp.flags & KAON_F_GC) && T.factored;
   const bool coupled = (hp.flags & KAON_F_PD_COUPLED) != 0;
   const float tgb = rbf(hp.pd_tg);
@@ -1005,7 +1004,7 @@ __global__ __launch_bounds__(KAON_WG) void k_pd1(const KaonTensor* __restrict__ 
         const int cnt = chunk_cnt(c, C);
         if (cnt <= 0) continue;
         float x[8];
-        ld8<GT>(T.g, r * C + c * 8, cnt, vec && cnt == 8, x);
+        ld8<GT>(T.g, r * C + c * 8, cnt, r * C + c * 8 + 8 <= T.n, x);
 #pragma unroll
         for (int i = 0; i < 8; ++i)
           if (i < cnt) a = a + x[i];
@@ -1022,9 +1021,10 @@ __global__ __launch_bounds__(KAON_WG) void k_pd1(const KaonTensor* __restrict__ 
       const int cnt = chunk_cnt(c, C);
       if (cnt <= 0) continue;
       const int64_t e0 = r * C + c * 8;
-      const bool vv = vec && cnt == 8;
+      // a row's partial last chunk reads on into the next row (not past the tensor)
+      const bool vv = cnt == 8, vl = e0 + 8 <= T.n;
       float g[8];
-      ld8<GT>(T.g, e0, cnt, vv, g);
+      ld8<GT>(T.g, e0, cnt, vl, g);
       if (gc) {
 #pragma unroll
         for (int i = 0; i < 8; i += 2) {
@@ -1036,13 +1036,13 @@ __global__ __launch_bounds__(KAON_WG) void k_pd1(const KaonTensor* __restrict__ 
       }
       if (coupled) {
         float p[8];
-        ld8<PT>(T.p, e0, cnt, vv, p);
+        ld8<PT>(T.p, e0, cnt, vl, p);
 #pragma unroll
         for (int i = 0; i < 8; ++i) g[i] = __fmaf_rn(hp.wdl, p[i], g[i]);
       }
       if (CODEC != KAON_MOM_NONE) {
         uint32_t mq[8];
-        ld_mom_at<CODEC>(T.m, e0, cnt, vv, mq);
+        ld_mom_at<CODEC>(T.m, e0, cnt, vl, mq);
         if (CODEC == KAON_MOM_F32 || CODEC == KAON_MOM_BF16) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
@@ -1084,7 +1084,7 @@ __global__ __launch_bounds__(KAON_WG) void k_pd1(const KaonTensor* __restrict__ 
       }
       if (T.full_v) {
         float v[8];
-        ld8<KAON_F32>(T.v, e0, cnt, vv, v);
+        ld8<KAON_F32>(T.v, e0, cnt, vl, v);
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = __fmaf_rn(hp.pd_vval * g[i], g[i], v[i] * hp.b2);
         st8_f32(T.v, e0, cnt, vv, v);
@@ -1327,7 +1327,6 @@ __global__ __launch_bounds__(KAON_WG) void k_pd2(const KaonTensor* __restrict__ 
   const int64_t C = T.C, n = T.n;
   const int64_t nch = (C + 7) >> 3;
   const int cpl = (int)((nch + 63) >> 6);
-  const bool vec_t = T.vec_rows != 0;
   const bool gc = (hp.flags & KAON_F_GC) && T.factored;
   const bool cautious = (hp.flags & KAON_F_CAUTIOUS) != 0;
   const bool decoupled_wd = (hp.flags & KAON_F_WD) != 0;
@@ -1365,24 +1364,25 @@ __global__ __launch_bounds__(KAON_WG) void k_pd2(const KaonTensor* __restrict__ 
       if (cnt <= 0) continue;
       const int64_t j0 = c * 8;
       const int64_t e0 = r * C + j0;
-      const bool vec = vec_t && cnt == 8;
+      // a row's partial last chunk reads on into the next row (not past the tensor)
+      const bool vec = cnt == 8, vl = e0 + 8 <= n;
       float g[8], p[8], f[8];
       uint32_t mq[8], pb[8];
-      ld8<GT>(T.g, e0, cnt, vec, g);
+      ld8<GT>(T.g, e0, cnt, vl, g);
       const bool need_p = PHASE == 6 || decoupled_wd || (coupled && (CODEC == KAON_MOM_INT8 || CODEC == KAON_MOM_4BIT));
       if (need_p) {
         if (PT != KAON_F32) {
-          ld8_bits(T.p, e0, cnt, vec, pb);
+          ld8_bits(T.p, e0, cnt, vl, pb);
 #pragma unroll
           for (int i = 0; i < 8; ++i) p[i] = lp2f<PT>(pb[i]);
         } else {
-          ld8<KAON_F32>(T.p, e0, cnt, vec, p);
+          ld8<KAON_F32>(T.p, e0, cnt, vl, p);
         }
       } else {
 #pragma unroll
         for (int i = 0; i < 8; ++i) p[i] = 0.0f;
       }
-      if (CODEC != KAON_MOM_NONE) ld_mom_at<CODEC>(T.m, e0, cnt, vec, mq);
+      if (CODEC != KAON_MOM_NONE) ld_mom_at<CODEC>(T.m, e0, cnt, vl, mq);
       if (factored && T.fb_r) {
         // r c of each element's [fb_r, fb_c] block (n < 2^31: 32-bit indices)
         const uint32_t Rb = (uint32_t)T.fb_r, Cb = (uint32_t)T.fb_c, bsz = Rb * Cb;
@@ -1395,16 +1395,13 @@ __global__ __launch_bounds__(KAON_WG) void k_pd2(const KaonTensor* __restrict__ 
           f[i] = rfb[b * Rb + a] * cfb[b * Cb + c];
         }
       } else if (factored) {
-        ld8<KAON_F32>((const float*)ws.cf(T), j0, cnt, vec, f);
+        ld8<KAON_F32>((const float*)ws.cf(T), j0, cnt, true, f);  // C + 8 words
       } else {
-        ld8<KAON_F32>(T.v, e0, cnt, vec, f);
+        ld8<KAON_F32>(T.v, e0, cnt, vl, f);
       }
       uint32_t nz[8];
       if (PHASE == 6 && lowp && hp.bf16_method == KAON_SR) {
-        if ((e0 & 7) == 0) noise8(hp.seed, hp.step, (uint32_t)T.tensor_id, 1u, e0, T.noise[1], cnt, nz);
-        else
-#pragma unroll
-          for (int i = 0; i < 8; ++i) nz[i] = i < cnt ? noise1(hp.seed, hp.step, T.tensor_id, 1u, e0 + i, T.noise[1]) : 0u;
+        noise8_any(hp.seed, hp.step, (uint32_t)T.tensor_id, 1u, e0, T.noise[1], cnt, nz);
       }
       if (gc) {
 #pragma unroll
@@ -1496,7 +1493,7 @@ __global__ __launch_bounds__(KAON_WG) void k_pd2(const KaonTensor* __restrict__ 
         uint32_t o[8];
         if (hp.bf16_method == KAON_KAHAN) {
           uint32_t sh[8];
-          ld8_bits(T.shift, e0, cnt, vec, sh);
+          ld8_bits(T.shift, e0, cnt, vl, sh);
 #pragma unroll
           for (int i = 0; i < 8; ++i) {
             // shift -= lp(delta); p0 = p; p += shift; shift += p0 - p, in the
@@ -1549,14 +1546,13 @@ __global__ __launch_bounds__(KAON_WG) void k_gc_write(const KaonTensor* __restri
   const KaonTensor& T = D[it.tensor];
   if (!T.factored || T.n == 0 || !T.gc_write) return;
   const int64_t C = T.C, nch = (C + 7) >> 3;
-  const bool vec = T.vec_rows != 0;
   const WaveRows wr = wave_rows(it);
   for (int64_t r = wr.rb; r < wr.re; ++r) {
     const float mu = uniform_f(ws.mu(T)[r]);
     for (int64_t c = wr.lane; c < nch; c += 64) {
       const int cnt = chunk_cnt(c, C);
       const int64_t e0 = r * C + c * 8;
-      const bool vv = vec && cnt == 8;
+      const bool vv = cnt == 8;
       float x[8];
       ld8<GT>(T.g, e0, cnt, vv, x);
       if (GT != KAON_F32) {

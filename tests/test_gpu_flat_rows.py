@@ -88,3 +88,48 @@ def test_unaligned_storage_gives_the_same_bits(name):
         for k in sa:
             if torch.is_tensor(sa[k]):
                 assert np.array_equal(to_bits(sa[k]).reshape(-1), to_bits(sb[k]).reshape(-1)), k
+
+
+# rows whose chunks start at every offset, with partial last chunks, for the kernels that
+# walk rows with unaligned 16-byte accesses (KProdigy's passes, AdaMuon's momentum, MSAM's
+# norm); AdaMuon's orthogonalized update is compared between the two storages instead
+ROWS = [[5, 3], [41, 15], [9, 513], [43, 771], [6, 1029], [3, 520], [70], [2, 9, 5]]
+
+
+@pytest.mark.parametrize("mom,p,method,kw", [
+    ("bfloat16", "bf16", "stochastic_rounding", {}),
+    ("int8", "bf16", "stochastic_rounding", dict(second_moment="factored", weight_decay=0.01)),
+    ("4bit", "bf16", "kahan", dict(momentum_4bit_block=24)),
+    ("float32", "f32", "none", dict(second_moment="factored", cautious=True)),
+    ("int8", "f16", "none", {}),
+    ("bfloat16", "bf16", "none", dict(weight_decay=0.01, decouple=False)),
+])
+def test_kprodigy_rows_of_any_length_bit_exact(mom, p, method, kw):
+    case = dict(steps=3, seed=16, p_dtype=p, g_dtype=p, opt="kprodigy", shapes=ROWS,
+                kwargs=dict(lr=1.0, momentum_dtype=mom, bf16_method=method, **kw))
+    print(f"[gpu] kprodigy rows {mom} {p} {method}", flush=True)
+    oparams, _, _ = oracle_case_run(case)
+    params, gopt, _ = run_gpu(case)
+    assert_same_as_oracle(case, oparams, params, gopt, label=f"pd_{mom}")
+
+
+@pytest.mark.parametrize("mom", ["int8", "bfloat16"])
+def test_msam_and_adamuon_unaligned_rows(mom):
+    """MSAM's momentum norm against the oracle, and AdaMuon's momentum (codes, scales)."""
+    case = dict(steps=2, seed=17, p_dtype="bf16", g_dtype="bf16", opt="msam", shapes=ROWS,
+                kwargs=dict(lr=1e-3, momentum_dtype=mom))
+    print(f"[gpu] msam rows {mom}", flush=True)
+    oparams, _, _ = oracle_case_run(case)
+    params, gopt, _ = run_gpu(case)
+    assert_same_as_oracle(case, oparams, params, gopt, label=f"msam_{mom}")
+    case = dict(steps=1, seed=18, p_dtype="bf16", g_dtype="bf16", opt="adamuon", shapes=[[9, 513], [43, 71], [16, 33]],
+                kwargs=dict(lr=1e-3, momentum_dtype=mom))
+    oparams, _, _ = oracle_case_run(case)
+    params, gopt, _ = run_gpu(case)
+    for op, prm in zip(oparams, params):
+        for k in ("m", "m_scale"):
+            if k in op.state:
+                got = to_bits(state_of(gopt, prm)[k]).reshape(-1)
+                want = np.asarray(op.state[k]).reshape(-1)
+                want = want.view(got.dtype) if want.itemsize == got.itemsize else want
+                assert np.array_equal(got, want), k
