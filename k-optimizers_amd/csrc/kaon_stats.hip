@@ -633,7 +633,7 @@ __device__ __forceinline__ void pf_stats_body(const KaonTensor& T, const KaonIte
       seg_put(sbuf(0, k), wr.w, wr.lane, v);
     }
     if (k % SEGG == SEGG - 1 || k == CPL - 1) {
-      __syncthreads();
+      lds_barrier();  // only LDS is handed over; run partials stay with their thread
 #pragma unroll
       for (int kk = k - k % SEGG; kk <= k; ++kk)
         seg_fold<RAG>(sbuf(0, kk), nw, (int64_t)kk * 512, C, part, acc, last, tid, racc);
@@ -674,7 +674,7 @@ __device__ __forceinline__ void pf_stats_body(const KaonTensor& T, const KaonIte
       seg_put(sbuf(1, k), wr.w, wr.lane, v);
     }
     if (k % SEGG == SEGG - 1 || k == CPL - 1) {
-      __syncthreads();
+      lds_barrier();
 #pragma unroll
       for (int kk = k - k % SEGG; kk <= k; ++kk) {
         if (REG2)
@@ -731,7 +731,7 @@ __device__ __forceinline__ void pf_stats_run(const KaonTensor& T, const KaonItem
   for (int i = 0; i < 48; ++i) rr2[i] = 0.0f;
 #pragma clang loop unroll(disable)
   for (int sl = 0; sl < nsl; ++sl) {
-    if (sl > 0) __syncthreads();  // the LDS fold buffers are reused
+    if (sl > 0) lds_barrier();  // the LDS fold buffers are reused
     const KaonItem si = slice_item(it, sl);
     KAON_PF_SWITCH(CLS, pf_stats_body, KAON_COMMA GT KAON_COMMA EPS KAON_COMMA REG2 KAON_COMMA RAG, T, si, ws, hp, mode,
                    seg, part, sl > 0, sl + 1 == nsl, racc, part2, racc2, rr2)

@@ -2229,9 +2229,9 @@ int kaon_kprodigy_pass1(const KaonLaunch* L, const KaonHyper* hp, void* stream) 
   if (!f1 || !fs) return fail("kaon_kprodigy_pass1: unsupported dtype / codec combination");
   hipLaunchKernelGGL(k_pd_zero, dim3(L->n_tensors), dim3(KAON_WG), 0, st, L->descs, ws, codec);
   if ((rc = check_launch("kaon: KProdigy zero launch"))) return rc;
-  // the factored row/col EMAs (tensors with a per-element v return at once)
-  if ((rc = run_stats(*L, ws, h, 0, st))) return rc;
+  // the factored row/col EMAs (every 1-D tensor has a per-element v)
   if (L->n_fin_items > 0) {
+    if ((rc = run_stats(*L, ws, h, 0, st))) return rc;
     hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, h);
     if ((rc = check_launch("kaon: k_fin launch"))) return rc;
   }

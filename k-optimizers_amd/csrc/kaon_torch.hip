@@ -439,15 +439,6 @@ __device__ __forceinline__ float tclip_u(const KaonTensor& T, const Ws& ws, int6
   return (xg * ws.rf(T)[r]) * ws.cf(T)[j];
 }
 
-// Workgroup barrier that orders LDS only.  __syncthreads() also fences global
-// memory, which waits for every load in flight -- the producers' loads issued
-// blocks ahead included; the block handoff needs only the LDS writes done.
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
-
 // A producer slot's raw loads for one chunk: the grad chunk (16-bit grads kept
 // packed, two to a word), the column factors (or v), the row's GC mean and factor.
 template <int GT>
