@@ -78,10 +78,11 @@ int check_launch(const char* what) {
 // columns (and of both partials) before it adds the current one; kind 1 has the
 // four waves load 8 rounds of rows into LDS at a time for the one wave that adds.
 // One load batch after the other took 160-180 us for that embedding's net (124 M
-// params), this 68 us; 405 matrices of a UNet (677 M) 75 -> 37 us.
-template <int NC>
+// params), this 68 us with 256 threads and 46 us with 1024 (launch_fin); 405 matrices
+// of a UNet (677 M) 75 -> 37 us with 256.
+template <int NC, int WG>
 __device__ __forceinline__ float fin_cols(const KaonTensor& T, const KaonItem& it, const Ws& ws, const KaonHyper& hp,
-                                          bool alg) {
+                                          bool alg, float* quot) {
   constexpr int U = NC == 1 ? 12 : NC == 2 ? 8 : NC == 3 ? 6 : NC <= 5 ? 4 : 2;  // runs per batch
   const int64_t C = T.C;
   const int ng = T.ngroups;
@@ -96,7 +97,7 @@ __device__ __forceinline__ float fin_cols(const KaonTensor& T, const KaonItem& i
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     // threads past the item's columns read its last one
-    j[c] = min((int64_t)it.row0 + (int)threadIdx.x + KAON_WG * c, jend - 1);
+    j[c] = min((int64_t)it.row0 + (int)threadIdx.x + WG * c, jend - 1);
     cs[c] = c2[c] = 0.0f;
     old[c] = T.col[j[c]];
   }
@@ -146,35 +147,56 @@ __device__ __forceinline__ float fin_cols(const KaonTensor& T, const KaonItem& i
   float a = 0.0f;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    if ((int64_t)it.row0 + (int)threadIdx.x + KAON_WG * c >= jend) continue;
+    if ((int64_t)it.row0 + (int)threadIdx.x + WG * c >= jend) continue;
     const float nc = klerp(old[c], cs[c] / fR, hp.w2);
     T.col[j[c]] = nc;
     put_cf(cf, C, j[c], 1.0f / sqrtf(nc));
-    if (alg) a = a + c2[c] / nc;
+    if (WG != KAON_WG) quot[threadIdx.x + WG * c] = c2[c] / nc;
+    else if (alg) a = a + c2[c] / nc;
+  }
+  if (WG != KAON_WG && alg) {
+    // thread t < 256 adds the columns t, t + 256, ... as the narrow workgroup does
+    __syncthreads();
+    if (threadIdx.x < KAON_WG)
+      for (int k = threadIdx.x; k < it.nrows; k += KAON_WG) a = a + quot[k];
   }
   return a;
 }
-__global__ __launch_bounds__(KAON_WG, 4) void k_fin(const KaonTensor* __restrict__ D,
-                                                 const KaonItem* __restrict__ items, Ws ws, KaonHyper hp) {
+template <int WG>
+__global__ __launch_bounds__(WG, 4) void k_fin(const KaonTensor* __restrict__ D, const KaonItem* __restrict__ items,
+                                               Ws ws, KaonHyper hp) {
   constexpr int kRounds = 8;  // rounds of 64 chunks of rows in LDS
-  __shared__ float rows[kRounds * 512];
+  constexpr int kLd = kRounds * 512 / WG;
+  __shared__ __attribute__((aligned(16))) float rows[kRounds * 512];  // kind 0: the columns' quotients
   __shared__ float rm_s;
-  __shared__ float red4[4];
+  __shared__ float red4[WG / 64];
   const KaonItem it = items[blockIdx.x];
   const KaonTensor& T = D[it.tensor];
   const int64_t R = T.R;
   if (it.kind == 0) {
     const bool alg = clip_alg(hp, 0);
     float a = 0.0f;
-    switch ((it.nrows + KAON_WG - 1) / KAON_WG) {
-      case 1: a = fin_cols<1>(T, it, ws, hp, alg); break;
-      case 2: a = fin_cols<2>(T, it, ws, hp, alg); break;
-      case 3: a = fin_cols<3>(T, it, ws, hp, alg); break;
-      case 4: a = fin_cols<4>(T, it, ws, hp, alg); break;
-      case 5: a = fin_cols<5>(T, it, ws, hp, alg); break;
-      case 6: a = fin_cols<6>(T, it, ws, hp, alg); break;
-      case 7: a = fin_cols<7>(T, it, ws, hp, alg); break;
-      case 8: a = fin_cols<8>(T, it, ws, hp, alg); break;
+    switch ((it.nrows + WG - 1) / WG) {
+      case 1: a = fin_cols<1, WG>(T, it, ws, hp, alg, rows); break;
+      case 2: a = fin_cols<2, WG>(T, it, ws, hp, alg, rows); break;
+      case 3:
+        if constexpr (3 * WG <= KAON_COLITEM) a = fin_cols<3, WG>(T, it, ws, hp, alg, rows);
+        break;
+      case 4:
+        if constexpr (4 * WG <= KAON_COLITEM) a = fin_cols<4, WG>(T, it, ws, hp, alg, rows);
+        break;
+      case 5:
+        if constexpr (5 * WG <= KAON_COLITEM) a = fin_cols<5, WG>(T, it, ws, hp, alg, rows);
+        break;
+      case 6:
+        if constexpr (6 * WG <= KAON_COLITEM) a = fin_cols<6, WG>(T, it, ws, hp, alg, rows);
+        break;
+      case 7:
+        if constexpr (7 * WG <= KAON_COLITEM) a = fin_cols<7, WG>(T, it, ws, hp, alg, rows);
+        break;
+      case 8:
+        if constexpr (8 * WG <= KAON_COLITEM) a = fin_cols<8, WG>(T, it, ws, hp, alg, rows);
+        break;
     }
     if (alg) {
       const float S = wg_sum4(a, red4);
@@ -183,12 +205,26 @@ __global__ __launch_bounds__(KAON_WG, 4) void k_fin(const KaonTensor* __restrict
   } else {
     const KAON_G float* row = G(T.row);
     float a = 0.0f;
+    // the wide workgroup loads the next rounds while its first wave adds (the narrow
+    // one has no registers for them: it spilled)
+    constexpr bool kAhead = WG > KAON_WG;
+    float nx[kLd];
     for (int64_t r0 = 0; r0 < R; r0 += kRounds * 512) {
       const int nr = (int)min<int64_t>(kRounds * 512, R - r0);
       if (r0 > 0) __syncthreads();  // the rows are written again
-#pragma unroll 16
-      for (int k = threadIdx.x; k < nr; k += KAON_WG) rows[k] = row[r0 + k];
+      if (!kAhead || r0 == 0) {
+#pragma unroll kLd
+        for (int k = threadIdx.x; k < nr; k += WG) rows[k] = row[r0 + k];
+      } else {
+#pragma unroll
+        for (int u = 0; u < kLd; ++u) rows[threadIdx.x + u * WG] = nx[u];
+      }
       __syncthreads();
+      if (kAhead && r0 + kRounds * 512 < R) {
+#pragma unroll
+        for (int u = 0; u < kLd; ++u)
+          nx[u] = row[min(r0 + kRounds * 512 + (int)threadIdx.x + u * WG, R - 1)];
+      }
       if (threadIdx.x < 64) {
         for (int e = 8 * (int)threadIdx.x; e < nr; e += 512) {
           if (e + 8 <= nr) {
@@ -211,15 +247,29 @@ __global__ __launch_bounds__(KAON_WG, 4) void k_fin(const KaonTensor* __restrict
     __syncthreads();
     const double rrm = rcp64(rm_s);  // exact quotients (div_r64)
     KAON_G float* rf = ws.rf(T);
-    for (int64_t i0 = threadIdx.x; i0 < R; i0 += 16 * KAON_WG) {
-      float v[16];
+    for (int64_t i0 = threadIdx.x; i0 < R; i0 += kLd * WG) {
+      float v[kLd];
 #pragma unroll
-      for (int u = 0; u < 16; ++u) v[u] = row[min(i0 + u * KAON_WG, R - 1)];
+      for (int u = 0; u < kLd; ++u) v[u] = row[min(i0 + u * WG, R - 1)];
 #pragma unroll
-      for (int u = 0; u < 16; ++u)
-        if (i0 + u * KAON_WG < R) rf[i0 + u * KAON_WG] = 1.0f / sqrtf(div_r64(v[u], rrm));
+      for (int u = 0; u < kLd; ++u)
+        if (i0 + u * WG < R) rf[i0 + u * WG] = 1.0f / sqrtf(div_r64(v[u], rrm));
     }
   }
+}
+
+// Workgroups of 1024 threads where the items are fewer than the chip holds of them
+// (two per CU) and the tensors mostly tall (several runs each): the largest item's
+// chain is then the launch, and four times the threads keep four times the loads in
+// flight (fp32 transformer of 124 M params: 68 -> 46 us, the step 898 -> 879; 52 M
+// params of odd dims: 340.4 -> 334.7).  More items fill the CUs with workgroups of
+// 256, and tensors of one run have nothing for the other waves to do.
+int launch_fin(const KaonLaunch& L, Ws ws, const KaonHyper& hp, hipStream_t st) {
+  constexpr int kWide = 1024;
+  const bool wide = L.n_fin_items <= 2 * 256 && L.n_row_items >= 2 * L.n_tensors;
+  hipLaunchKernelGGL(wide ? k_fin<kWide> : k_fin<KAON_WG>, dim3(L.n_fin_items), dim3(wide ? kWide : KAON_WG), 0, st,
+                     L.descs, L.fin_items, ws, hp);
+  return check_launch("kaon: k_fin launch");
 }
 
 // =============================================================== phase 4
@@ -2035,8 +2085,7 @@ int kaon_adakaon_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask,
       if ((rc = run_stats(*L, ws, h, 0, st))) return rc;
     }
     if ((mask & (1u << 2)) && L->n_fin_items > 0) {
-      hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, h);
-      if ((rc = check_launch("kaon: k_fin launch"))) return rc;
+      if ((rc = launch_fin(*L, ws, h, st))) return rc;
     }
     // phase 3 (the clip's sum of squares) is folded into phases 1 and 2, phase 4 (its
     // divisor) into phases 5 and 6
@@ -2090,8 +2139,7 @@ int kaon_adamuon_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask,
     if ((rc = run_stats(*L, ws, ho, 0, st))) return rc;
   }
   if ((mask & (1u << 2)) && L->n_fin_items > 0) {
-    hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, ho);
-    if ((rc = check_launch("kaon: k_fin launch"))) return rc;
+    if ((rc = launch_fin(*L, ws, ho, st))) return rc;
   }
   // phase 3 (the clip's sum of squares) is folded into phases 1 and 2, phase 4 (its
   // divisor) into phases 5 and 6
@@ -2129,8 +2177,7 @@ int kaon_adapnm_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask, 
     if ((rc = run_stats(*L, ws, h, 0, st))) return rc;
   }
   if ((mask & (1u << 2)) && L->n_fin_items > 0) {
-    hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, h);
-    if ((rc = check_launch("kaon: k_fin launch"))) return rc;
+    if ((rc = launch_fin(*L, ws, h, st))) return rc;
   }
   if (mask & (1u << 3)) {
     // row class 0 (the leading row items) with int8 / bf16 momenta: the prefetching kernel
@@ -2232,8 +2279,7 @@ int kaon_kprodigy_pass1(const KaonLaunch* L, const KaonHyper* hp, void* stream) 
   // the factored row/col EMAs (every 1-D tensor has a per-element v)
   if (L->n_fin_items > 0) {
     if ((rc = run_stats(*L, ws, h, 0, st))) return rc;
-    hipLaunchKernelGGL(k_fin, dim3(L->n_fin_items), dim3(KAON_WG), 0, st, L->descs, L->fin_items, ws, h);
-    if ((rc = check_launch("kaon: k_fin launch"))) return rc;
+    if ((rc = launch_fin(*L, ws, h, st))) return rc;
   }
   hipLaunchKernelGGL(f1, dim3(L->n_row_items), dim3(KAON_WG), 0, st, L->descs, L->row_items, ws, h);
   if ((rc = check_launch("kaon: KProdigy pass-1 launch"))) return rc;

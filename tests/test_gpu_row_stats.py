@@ -16,11 +16,14 @@ LONG = [[3, 129], [85, 137], [21, 511], [41, 513], [13, 1025], [5, 2047], [6, 20
 # many runs per column (the finalize step's batches of partials, 1 to 8 columns per thread)
 # and many rounds of rows for the row factors' mean
 TALL = [[5001, 70], [9000, 9], [4097, 300], [40000, 3], [700, 520], [333, 1100], [50, 2049], [40, 5000], [4100, 16]]
+# the same among many short tensors: the finalize step's narrow workgroups
+MANY = TALL + [[3, 5]] * 200
 # whole 16-byte rows of fewer than 8 chunks: 1 to 7 chunks, several rows side by side
 THIN = [[300, 16], [77, 8], [90, 24], [50, 40], [33, 64], [641, 32], [25, 56], [96, 48]]
 
 CASES = {
     "bf16_tall": ("adakaon", TALL, dict(momentum_dtype="int8", clip_threshold=0.05), "bf16", "bf16"),
+    "bf16_tall_many": ("adakaon", MANY, dict(momentum_dtype="int8", clip_threshold=0.05), "bf16", "bf16"),
     "f32_tall": ("adakaon", TALL, dict(), "f32", "f32"),
     "pnm_tall": ("adapnm", TALL[:4], dict(momentum_dtype="int8"), "bf16", "bf16"),
     "thin_int8": ("adakaon", THIN, dict(momentum_dtype="int8", weight_decay=0.02), "bf16", "bf16"),
