@@ -32,22 +32,23 @@ constexpr int mom_words() {
   return CODEC == KAON_MOM_F32 ? 8 : CODEC == KAON_MOM_BF16 ? 4 : CODEC == KAON_MOM_INT8 ? 2 : 1;
 }
 
-// NW words at a chunk's address: 16-, 8- or 4-byte accesses when `vec` (the
-// tensor's bases are 16-byte aligned and the chunk is whole), otherwise byte by
-// byte, `nbytes` of them (the rest reads as 0 / is not written).
+// NW words at a chunk's address, at any alignment: 16-, 8- or 4-byte accesses when
+// `vec` (the chunk is whole), otherwise byte by byte, `nbytes` of them (the rest
+// reads as 0 / is not written).
 template <int NW>
 __device__ __forceinline__ void ld_words(const KAON_G uint8_t* a, bool vec, int nbytes, uint32_t (&w)[NW]) {
   if (vec) {
     if constexpr (NW == 1) {
-      w[0] = ld_stream<true>((const KAON_G uint32_t*)a);
+      w[0] = __builtin_nontemporal_load((const KAON_G ku1_any*)a);
     } else if constexpr (NW == 2) {
-      const ku2 v = ld_stream<true>((const KAON_G ku2*)a);
+      const ku2 v = __builtin_nontemporal_load((const KAON_G ku2_any*)a);
       w[0] = v.x;
       w[1] = v.y;
     } else {
 #pragma unroll
       for (int k = 0; k < NW / 4; ++k) {
-        const ku4 v = ld_stream<NW == 4>((const KAON_G ku4*)a + k);
+        const KAON_G ku4_any* q = (const KAON_G ku4_any*)a + k;
+        const ku4 v = NW == 4 ? __builtin_nontemporal_load(q) : *q;
         w[4 * k] = v.x;
         w[4 * k + 1] = v.y;
         w[4 * k + 2] = v.z;
@@ -68,14 +69,16 @@ template <int NW>
 __device__ __forceinline__ void st_words(KAON_G uint8_t* a, bool vec, int nbytes, const uint32_t (&w)[NW]) {
   if (vec) {
     if constexpr (NW == 1) {
-      st_stream((KAON_G uint32_t*)a, w[0]);
+      __builtin_nontemporal_store(w[0], (KAON_G ku1_any*)a);
     } else if constexpr (NW == 2) {
-      st_stream((KAON_G ku2*)a, ku2{w[0], w[1]});
+      __builtin_nontemporal_store(ku2{w[0], w[1]}, (KAON_G ku2_any*)a);
     } else {
 #pragma unroll
-      for (int k = 0; k < NW / 4; ++k)
-        if (NW == 4) st_stream((KAON_G ku4*)a + k, ku4{w[0], w[1], w[2], w[3]});
-        else ((KAON_G ku4*)a)[k] = ku4{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
+      for (int k = 0; k < NW / 4; ++k) {
+        const ku4 v = ku4{w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]};
+        if (NW == 4) __builtin_nontemporal_store(v, (KAON_G ku4_any*)a + k);
+        else ((KAON_G ku4_any*)a)[k] = v;
+      }
     }
     return;
   }
@@ -136,7 +139,7 @@ struct Pos {
   uint32_t lo;  // the chunk's first element in the window
   uint32_t r, j0;  // its row (relative to the slice) and column
   int cnt;      // existing elements (0 for a lane outside the slice)
-  bool vec;     // wave-uniform: whole chunks, aligned
+  bool vec;     // wave-uniform: whole chunks
 };
 
 // What a chunk reads from memory, loaded a window ahead of its arithmetic.
@@ -152,7 +155,7 @@ struct FlatCtx {
   const KAON_G uint8_t *msc, *nsc;  // scales of m (per row or block), of AdaPNM's negative buffer
   const uint16_t* nz[3];
   uint32_t tid;
-  bool factored, vec;
+  bool factored;
 };
 
 // Bytes of `cnt` (<= 8) elements of a momentum codec.
@@ -176,8 +179,7 @@ struct FlatCfg {
   static constexpr bool ABSMAX = PHASE == 5 && QUANT && MOM && !PNM && !MUON;
 };
 
-// VEC: the slice's chunks are whole and 16-byte aligned and the tensor is
-// factored, so that no load sits behind a branch: a load in a branch, or one
+// VEC: the slice's chunks are whole and the tensor is factored, so that no load sits behind a branch: a load in a branch, or one
 // whose successors are conditional, would make the compiler wait for every load
 // in flight at its use, the next window's included.
 template <int OPT, int PHASE, int PT, int GT, int CODEC, bool XF, bool VEC>
@@ -228,14 +230,19 @@ __device__ __forceinline__ void flat_load(FlatIn<OPT, PHASE, PT, GT, CODEC>& in,
 // (16 B/param) and 237 -> 138 us.  Rows of 771 and 2057 bf16 elements with int8
 // momentum, 52.2 M params: 420 -> 138 us and 263 -> 74 us (the row-by-row walk in
 // front of each arrow).  Streams of 32 bytes per chunk (fp32) are ordinary
-// accesses: two 16-byte halves with a stride of 32 as non-temporal stores cost
-// 578 us of the 490.  Phase 5 fits 4 waves per SIMD (128 VGPRs); the apply spills
+// accesses (the apply took 578 us with non-temporal stores of two 16-byte halves
+// with a stride of 32, 490 so).  Storage that is not 16-byte aligned takes the same
+// accesses (whole steps with the gradients one element into their storage, read
+// byte by byte before the arrow: fp32, 58 M params, 1313 -> 442 us, aligned 433;
+// bf16 kahan 1167 -> 431, aligned 391; the odd rows 765 -> 345, aligned 335; plain
+// instead of non-temporal accesses 462, 428 and 333, but 454, 405 and 321 aligned).
+// Phase 5 fits 4 waves per SIMD (128 VGPRs); the apply spills
 // there (int8 201 us), so it takes 3.
 template <int OPT, int PHASE, int PT, int GT, int CODEC, bool XF>
 __global__ __launch_bounds__(KAON_WG, PHASE == 5 ? 4 : 3) void k_flat(const KaonTensor* __restrict__ D,
                                                      const KaonItem* __restrict__ items, Ws ws, KaonHyper hp) {
   using F = FlatCfg<OPT, PHASE, CODEC, XF>;
-  constexpr bool PNM = F::PNM, MUON = F::MUON, LION = F::LION, INT8 = F::INT8, Q4 = F::Q4, QUANT = F::QUANT;
+  constexpr bool PNM = F::PNM, MUON = F::MUON, LION = F::LION, INT8 = F::INT8, Q4 = F::Q4;
   constexpr bool MOM = F::MOM, ABSMAX = F::ABSMAX, NEEDP = F::NEEDP, KAHAN = F::KAHAN;
   constexpr bool LOWP = PT == KAON_BF16;
   using In = FlatIn<OPT, PHASE, PT, GT, CODEC>;
@@ -279,7 +286,6 @@ __global__ __launch_bounds__(KAON_WG, PHASE == 5 ? 4 : 3) void k_flat(const Kaon
   for (int s = 0; s < 3; ++s) X.nz[s] = T.noise[s];
   X.tid = (uint32_t)T.tensor_id;
   X.factored = factored;
-  X.vec = T.vec_flat != 0;
 
   // the slice's chunks [cb, ce) and their windows of 64
   const int64_t ebeg = (int64_t)it.row0 * C;
@@ -295,7 +301,7 @@ __global__ __launch_bounds__(KAON_WG, PHASE == 5 ? 4 : 3) void k_flat(const Kaon
     const int cc = min(max(lane, lo), hi);
     q.lo = (uint32_t)cc << 3;
     q.cnt = (int)min<int64_t>(8, n - (q.wb + q.lo));
-    q.vec = X.vec && __builtin_amdgcn_ballot_w64(q.cnt < 8) == 0;
+    q.vec = __builtin_amdgcn_ballot_w64(q.cnt < 8) == 0;
     const uint32_t rel = (uint32_t)(q.wb - ebeg) + q.lo;
     if (it.nrows == 1) {
       q.r = 0u;
@@ -662,7 +668,7 @@ __global__ __launch_bounds__(KAON_WG, PHASE == 5 ? 4 : 3) void k_flat(const Kaon
   using Yes = std::integral_constant<bool, true>;
   using No = std::integral_constant<bool, false>;
   const int64_t first = w0 + w;
-  if (X.vec && factored && ce * 8 <= n) {
+  if (factored && ce * 8 <= n) {
     // each window's loads are issued inside the previous window's arithmetic,
     // into two buffers in turn (a copy would wait for the loads in flight)
     In buf0, buf1;
