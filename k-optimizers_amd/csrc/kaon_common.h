@@ -188,8 +188,8 @@ __device__ __forceinline__ float clip_div(const KaonTensor& T, const Ws& ws, con
 // (k_clipdiv) checks that minimum scaled by lr / fac against 2^-120 (far above the
 // rounding of d and d * g) and lr <= 1/2 (an uncounted product that underflowed
 // stays 0 when scaled down; fac >= 1).  A tensor that fails has its count cleared
-// and word 3 set, and only then does phase 5 count it.  NaN counts in neither form,
-// and a fac that is inf or NaN fails the check.  Two bf16 momenta, 677 M params:
+// and word 3 set, and only then does phase 5 count it.  NaN counts in neither form;
+// an infinite fac fails the check, and a NaN clip sum leaves fac at 1.  Two bf16 momenta, 677 M params:
 // the keep-count pass took 622 us (6 B/param read), its early exit takes 14 us and
 // the count adds 20 us to the clip-sum pass.
 struct KeepEarly {
@@ -201,24 +201,34 @@ struct KeepEarly {
     keep += k ? 1u : 0u;
     least = fminf(least, k ? fminf(fabsf(u), x) : least);
   }
-  // every thread of the workgroup calls it
-  __device__ __forceinline__ void flush(const KaonTensor& T, const Ws& ws) {
+  // Every thread of the workgroup calls it.  A slice of one wave group (it.kind rows)
+  // leaves the other waves without rows: its wave stores its own count, and the idle
+  // ones end at once.  Waiting for it they kept three of four wave slots (of one XCD:
+  // one-slice runs launch every 16th workgroup) through its rows: 512 tensors [16, 64],
+  // int8 29 us without the count, 63 so, 35 now; 4-bit 81, 159, 92.  Slices of more
+  // wave groups add theirs up first (a count per wave made 555 us of the 505 of an
+  // 81 M-parameter set's step, at one address per tensor).
+  __device__ __forceinline__ void flush(const KaonTensor& T, const KaonItem& it, const Ws& ws) {
     __shared__ uint32_t ks[4];
     __shared__ uint32_t ls[4];
     const uint32_t k = wave_sum_u32(keep);
     const uint32_t l = wave_butterfly(__float_as_uint(least), [](uint32_t a, uint32_t b) { return a < b ? a : b; });
+    if (it.nrows <= it.kind) {
+      if ((threadIdx.x & 63) == 0) store(T, ws, k, l);
+      return;
+    }
     if ((threadIdx.x & 63) == 0) {
       ks[threadIdx.x >> 6] = k;
       ls[threadIdx.x >> 6] = l;
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      const uint32_t tot = ks[0] + ks[1] + ks[2] + ks[3];
-      if (tot) {
-        atomicAdd(ws.keep_ctr(T), tot);
-        atomicMin(ws.keep_ctr(T) + 1, min(min(ls[0], ls[1]), min(ls[2], ls[3])));
-      }
-    }
+    if (threadIdx.x == 0)
+      store(T, ws, ks[0] + ks[1] + ks[2] + ks[3], min(min(ls[0], ls[1]), min(ls[2], ls[3])));
+  }
+  __device__ __forceinline__ static void store(const KaonTensor& T, const Ws& ws, uint32_t k, uint32_t l) {
+    if (!k) return;
+    atomicAdd(ws.keep_ctr(T), k);
+    atomicMin(ws.keep_ctr(T) + 1, l);
   }
 };
 // Whether phase 5 still has to count this AdaPNM tensor.

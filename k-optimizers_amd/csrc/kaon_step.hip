@@ -720,7 +720,7 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm(const KaonTensor* __restrict__ 
     if (wr.lane == 0) ws.rs(T)[r] = s2;
   }
   if (CODEC == KAON_MOM_4BIT) bm4.flush(ws.bamax(T));
-  if (hp.flags & KAON_F_CAUTIOUS) ke.flush(T, ws);
+  if (hp.flags & KAON_F_CAUTIOUS) ke.flush(T, it, ws);
 }
 
 // AdaPNM phase 3 on row class 0 (factored, bf16 g, 16-byte rows with
@@ -861,7 +861,7 @@ __global__ __launch_bounds__(KAON_WG) void k_pnm_ss(const KaonTensor* __restrict
   switch (cpl) {
     KAON_PNM_SS(1) KAON_PNM_SS(2) KAON_PNM_SS(3) KAON_PNM_SS(4)
   }
-  if (hp.flags & KAON_F_CAUTIOUS) ke.flush(T, ws);
+  if (hp.flags & KAON_F_CAUTIOUS) ke.flush(T, it, ws);
 #undef KAON_PNM_SS
 }
 
