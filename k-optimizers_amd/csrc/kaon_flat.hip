@@ -698,12 +698,18 @@ __global__ __launch_bounds__(KAON_WG, PHASE == 5 ? 4 : 3) void k_flat(const Kaon
   } else {
     load_rows();
     __syncthreads();
+    // a vector is one row: no lookups per element (200 vectors of 1280 and 200 of 77,
+    // int8: Lion's keep count 5.8 -> 5.3 us and apply 7.4 -> 6.9, Adakaon's 9.9 -> 9.5
+    // and 10.5 -> 10.1; four of 4 M elements, whole Adakaon steps 12.8 -> 10.6 ms)
+    const bool str = nctx > 1;
     for (int64_t win = first; win < wend; win += 4) {
       In in;
       const Pos q = locate(win);
       flat_load<OPT, PHASE, PT, GT, CODEC, XF, false>(in, X, q);
-      const kaon_f32x2 am = chunk(in, q, Yes{}, No{}, [] {});
-      take_max(q, true, am);
+      kaon_f32x2 am;
+      if (str) am = chunk(in, q, Yes{}, No{}, [] {});
+      else am = chunk(in, q, No{}, No{}, [] {});
+      take_max(q, str, am);
     }
   }
 

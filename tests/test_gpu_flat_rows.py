@@ -117,7 +117,7 @@ def test_unaligned_storage_gives_the_same_bits(name, off_p, off_g):
 @pytest.mark.parametrize("name", ["lion_f32", "ada_bf16_kahan", "ada_int8_sr"])
 def test_unaligned_storage_steps_at_the_aligned_rate(name):
     """The same bytes in the same 16-byte accesses: at most 1.5 times the aligned step (1.0 to
-    1.1 measured; reading them byte by byte took 2.3 to 3.0)."""
+    1.1 measured; reading them byte by byte took 1.9 to 3.3)."""
     opt, kw, p, g = STORAGE[name]
     case = dict(steps=1, seed=12, p_dtype=p, g_dtype=g, opt=opt, kwargs=dict(lr=1e-3, **kw),
                 shapes=[[2048, 3073], [2048, 2057], [1025, 4097]])
