@@ -9,11 +9,13 @@ centralize in-kernel and leave p.grad as it was (src/kaon/adakaon.py:387-409);
 the fused Adakaon still sends some params to its native path (fp16, convs with
 quantized momentum, beta1 = 0, bf16 without SR, one-block 4-bit matrices of odd
 width: _fused_partition, adakaon.py:437-468), whose p.grad it centralizes.
-The Adakaon / Lion apply (Nekaon's and MSAM's removal / climb applies
+The Adakaon / Lion / AdaPNM apply (Nekaon's and MSAM's removal / climb applies
 included) and KProdigy's pass 2 store the centralized gradient as they read it
-(KAON_F_GC_WRITE); AdaPNM and AdaMuon write it back after the step with
+(KAON_F_GC_WRITE); AdaMuon writes it back after the step with
 kaon_gc_writeback.  Checked against the oracle's bf16 GC, after the last of
-the case's steps (Nekaon and MSAM: the second, whose apply carries the removal).
+the case's steps (Nekaon and MSAM: the second, whose apply carries the removal);
+for every gradient dtype, row length and alignment against the row means as the
+oracle sums them.
 """
 import numpy as np
 import pytest
@@ -111,3 +113,40 @@ def test_fused_big_matrix_keeps_its_grad_and_the_step_is_unchanged():
     assert np.array_equal(out[True][1], to_bits(g))
     want = O.gc_bf16(to_bits(g).reshape(600, 300)).reshape(out[False][1].shape)
     assert np.array_equal(out[False][1], want)
+
+
+def _centralized(v, gd):
+    """g - mean over the fan-in of a float32 array in the grad dtype gd, as bits: the row sum
+    in the oracle's order, the mean and the difference rounded to gd."""
+    rnd = {"bf16": lambda x: O.bf16_to_f32(O.f32_to_bf16(x)), "f16": lambda x: O.f16_to_f32(O.f32_to_f16(x)),
+           "f32": lambda x: np.asarray(x, np.float32)}[gd]
+    x = rnd(np.ascontiguousarray(v, np.float32)).reshape(v.shape[0], -1)
+    mu = np.empty((x.shape[0], 1), np.float32)
+    for r in range(x.shape[0]):
+        row = np.ascontiguousarray(x[r])
+        mu[r] = np.float32(O.lib().ko_csum(row.ctypes.data, row.size)) / np.float32(row.size)
+    out = np.ascontiguousarray(x - rnd(mu).reshape(-1, 1), np.float32)
+    return {"bf16": O.f32_to_bf16, "f16": O.f32_to_f16, "f32": lambda a: a}[gd](out)
+
+
+@pytest.mark.parametrize("off", [0, 1])
+@pytest.mark.parametrize("gd", ["bf16", "f16", "f32"])
+@pytest.mark.parametrize("opt", ["adakaon", "lion", "adapnm"])
+def test_grad_of_any_row_length_after_step(opt, gd, off):
+    """Rows shorter than a chunk, chunks that cross rows and slices, partial last chunks."""
+    from test_gpu_flat_rows import SHAPES as ROWS
+    from test_gpu_flat_rows import storage_run
+
+    case = dict(steps=2, seed=19, p_dtype=gd, g_dtype=gd, opt=opt, shapes=ROWS,
+                kwargs=dict(lr=1e-3, momentum_dtype="int8"))
+    print(f"[gpu] grad rows {opt} {gd} {off}", flush=True)
+    params, _ = storage_run(case, off, off)
+    for i, p in enumerate(params):
+        raw = grad_values(case, i, case["steps"])
+        got = to_bits(p.grad).reshape(-1)
+        if raw.ndim >= 2:
+            want = _centralized(raw, gd)
+        else:
+            want = to_bits(torch.from_numpy(raw).to(p.dtype))
+        want = np.ascontiguousarray(want).reshape(-1)
+        assert np.array_equal(got.view(np.uint8), want.view(np.uint8)), (opt, gd, off, ROWS[i])
