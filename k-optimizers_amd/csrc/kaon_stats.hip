@@ -37,11 +37,11 @@ __device__ __forceinline__ void add_coupled_wd(const KaonTensor& T, const KaonHy
 
 // mode 0 (Adakaon): GC row mean (stored), row EMA of mean_C(G^2), column
 // partial of the slice (wave groups folded in order in LDS); 1-D tensors: v
-// EMA.  mode 1 (Lion): GC row means only.  CPL > 0 keeps a row of up to CPL
-// chunks per lane in registers; CPL == 0 streams the row from memory (used for
-// rows longer than 24 chunks per lane, fp32 grads with long rows, and 1-D).
-// With KAON_F_PD_COUPLED (KProdigy, factored, coupled decay) G is the decayed
-// gradient fma(wd, p, GC(g)); the GC mean is still the raw gradient's.
+// EMA.  mode 1 (Lion): GC row means only.  CPL == 0 streams the row from memory
+// (rows longer than 24 chunks per lane, fp32 and fp16 grads of more than 10, and
+// 1-D).  CPL > 0 keeps a row of up to CPL chunks per lane in registers: KProdigy's
+// coupled decay (KAON_F_PD_COUPLED, factored) of every shorter row.  There G is the
+// decayed gradient fma(wd, p, GC(g)); the GC mean is still the raw gradient's.
 template <int GT, int CPL>
 __global__ __launch_bounds__(KAON_WG) void k_stats(const KaonTensor* __restrict__ D,
                                                    const KaonItem* __restrict__ items, Ws ws, KaonHyper hp,
@@ -60,12 +60,15 @@ __global__ __launch_bounds__(KAON_WG) void k_stats(const KaonTensor* __restrict_
   const int cpl = (int)((nch + 63) >> 6);
   const bool vec = T.vec_rows != 0;
   const bool eps = (hp.flags & KAON_F_EPS) != 0;
-  const bool alg = clip_alg(hp, mode);
-  const bool cwd = mode == 0 && (hp.flags & KAON_F_PD_COUPLED) != 0;
+  if constexpr (CPL > 0) mode = 0;
+  const bool alg = CPL == 0 && clip_alg(hp, mode);  // KProdigy does not clip
+  const bool cwd = CPL > 0 || (mode == 0 && (hp.flags & KAON_F_PD_COUPLED) != 0);
 
-  if (!T.factored) {
-    if (mode == 0) stats_1d<GT>(T, gsrc, hp, alg ? ws.scal(T) : nullptr, red4);
-    return;
+  if constexpr (CPL == 0) {
+    if (!T.factored) {
+      if (mode == 0) stats_1d<GT>(T, gsrc, hp, alg ? ws.scal(T) : nullptr, red4);
+      return;
+    }
   }
 
   const bool gc = (hp.flags & KAON_F_GC) != 0;
@@ -268,12 +271,9 @@ __global__ __launch_bounds__(KAON_WG) void k_stats(const KaonTensor* __restrict_
   if (!alg) continue;
   // The clip's second column partial, t = (G * G) / row (the new row; no
   // eps1), in the same wave-group / slice / run order, the rows read again
-  // (this kernel serves the grad layouts outside the prefetching kernels'
-  // register budget).
   KAON_G float* part2 = part + (int64_t)T.ngroups * C;
-  const int64_t segC = CPL > 0 ? C : (int64_t)kSeg;
-  for (int64_t c0 = 0; c0 < C; c0 += segC) {
-    const int64_t c1 = min(C, c0 + segC);
+  for (int64_t c0 = 0; c0 < C; c0 += kSeg) {
+    const int64_t c1 = min(C, c0 + (int64_t)kSeg);
     for (int wf = 0; wf < 4; ++wf) {
       if (wr.w == wf && has_rows) {
         for (int64_t c = (c0 >> 3) + wr.lane; c * 8 < c1; c += 64) {
@@ -335,7 +335,6 @@ template <int GT>
 struct Raw {
   uint32_t w[gt_words<GT>()];
 };
-typedef ku4 ku4_any __attribute__((aligned(2)));
 
 template <int GT, bool RAG>
 __device__ __forceinline__ void ld_raw(Raw<GT>& v, const KAON_G uint8_t* a) {
@@ -951,9 +950,9 @@ __global__ __launch_bounds__(KAON_WG) void k_pf_stats_wide(const KaonTensor* __r
   if (!stats_begin(T, it, ws, hp)) return;
   pf_stats_run<2, KAON_BF16, EPS, true, false>(T, it, ws, hp, mode, seg, racc, nullptr);
 }
-// Lion's row means alone (mode 1): the rows' loads and one butterfly each, without the
-// sums' registers and LDS.  The UNet set (2.66 G params): class 0 622 us in the kernel
-// above, 595 here; the Lion step 7460 -> 7425 us.
+// Lion's row means alone (mode 1): the rows' loads and one butterfly each.  The UNet set
+// (2.66 G params): class 0 takes 622 us in the kernel above, where the registers and LDS
+// of the sums and of the short rows are held too, 595 here.
 template <int CLS>
 __global__ __launch_bounds__(KAON_WG, CLS == 2 ? 2 : 4) void k_pf_mean(
     const KaonTensor* __restrict__ D, const KaonItem* __restrict__ items, Ws ws, KaonHyper hp, int) {
@@ -1025,12 +1024,15 @@ StatsFn pf_fn(int cls, bool fused) {
   return nullptr;
 }
 StatsFn mean_fn(int cls) { return cls == 0 ? k_pf_mean<0> : cls == 1 ? k_pf_mean<1> : k_pf_mean<2>; }
+// The register variants (classes 3-5) only for KProdigy's coupled decay.
 template <int GT>
 StatsFn streamed_fn(int cls) {
   switch (cls) {
     case 3: return k_stats<GT, 4>;
     case 4: return k_stats<GT, 10>;
-    case 5: return k_stats<GT, 24>;
+    case 5:  // planned for bf16 gradients only
+      if constexpr (GT == KAON_BF16) return k_stats<GT, 24>;
+      return nullptr;
     case 6: return k_stats<GT, 0>;
   }
   return nullptr;

@@ -19,10 +19,13 @@
 // wave-local butterfly with no LDS or barrier, and per-row values are
 // wave-uniform.  The tensor-global dependencies (column factors, row-mean,
 // clip divisor, cautious keep-count) split one step into launches:
-//   phase 1  slices      GC row means, row EMA, column partials (LDS fold)
-//   phase 2  fin items   column EMA + column factors; row mean + row factors
-//   phase 3  slices      per-row sums of U^2 (U = G*r*c)
-//   phase 4  tensors     clip divisor from the row sums
+//   phase 1  slices      GC row means, row EMA, column partials of G^2 and of the
+//                        clip's G^2 / row (LDS fold)
+//   phase 2  fin items   column EMA + column factors, the clip's item sums; row
+//                        mean + row factors
+//   phase 3  slices      AdaPNM only: per-row sums of U^2, the early keep count
+//   phase 4  tensors     AdaPNM only: clip divisor from the row sums (Adakaon and
+//                        AdaMuon form it in phases 5 and 6, clip_div)
 //   phase 5  slices      cautious keep-count, momentum absmax
 //   phase 6  slices      requant + momentum write, cautious rescale, weight
 //                        write (SR / RN / kahan / fp32), Nekaon remove+climb
@@ -151,8 +154,9 @@ __device__ __forceinline__ float fin_cols(const KaonTensor& T, const KaonItem& i
     const float nc = klerp(old[c], cs[c] / fR, hp.w2);
     T.col[j[c]] = nc;
     put_cf(cf, C, j[c], 1.0f / sqrtf(nc));
+    if (!alg) continue;
     if (WG != KAON_WG) quot[threadIdx.x + WG * c] = c2[c] / nc;
-    else if (alg) a = a + c2[c] / nc;
+    else a = a + c2[c] / nc;
   }
   if (WG != KAON_WG && alg) {
     // thread t < 256 adds the columns t, t + 256, ... as the narrow workgroup does
@@ -2271,6 +2275,7 @@ int kaon_kprodigy_pass1(const KaonLaunch* L, const KaonHyper* hp, void* stream) 
   const int codec = mom ? h.codec : KAON_MOM_NONE;
   h.codec = codec;
   h.flags &= ~(KAON_F_NK_REMOVE | KAON_F_NK_CLIMB | KAON_F_SRC_O | KAON_F_PNM);
+  h.clip = 0.0f;  // KProdigy does not clip: no clip sums in the row statistics
   PdFn f1 = pd1_fn(h.p_dtype, h.g_dtype, codec);
   PdStatsFn fs = pd_stats_fn(h.p_dtype, h.g_dtype);
   if (!f1 || !fs) return fail("kaon_kprodigy_pass1: unsupported dtype / codec combination");

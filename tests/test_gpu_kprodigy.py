@@ -90,6 +90,12 @@ EXTRA = {
     "factored_coupled": _case([[96, 48], [32, 16, 3, 3], [33, 45], [40, 1280], [6, 11520], [4, 20000], [77]],
                               dict(lr=1.0, second_moment="factored", momentum_dtype="int8", decouple=False,
                                    weight_decay=0.1, cautious=True), steps=3),
+    # the same past the first register class (rows of 2049 to 5120 columns) and, for fp32 / fp16
+    # gradients, past the second (streamed), whole and partial last chunks
+    **{f"factored_coupled_wide_{p}": _case([[6, 2056], [5, 4097], [9, 2049], [3, 5200]],
+                                           dict(lr=1.0, second_moment="factored", momentum_dtype="bfloat16",
+                                                decouple=False, weight_decay=0.1), steps=2, p=p, g=p)
+       for p in ("bf16", "f32", "f16")},
     # fp16 params and grads (RN under "stochastic_rounding", kahan in fp16): full and factored v
     "f16_full_sr": _case([[48, 40], [16, 8, 3, 3], [70]], dict(lr=1.0, momentum_dtype="int8", weight_decay=0.01,
                                                               cautious=True), p="f16", g="f16"),
