@@ -123,8 +123,9 @@ typedef struct KaonTensor {
                              and, for the RMS clip, of g^2 / row */
   int64_t ws_blk;         /* 4-bit: 2 arrays of nblocks words: amax, oldscale */
   int64_t ws_scal;        /* 5 + ceil(C / KAON_COLITEM) words (6 for 1-D): clip divisor, keep
-                             count, KProdigy num / den (MSAM / AdaMuon norms), mean(row), then
-                             the clip's partial sums, one per finalize item */
+                             count, KProdigy num / den (MSAM / AdaMuon norms; AdaPNM: the least
+                             counted product, whether phase 5 counts the tensor), mean(row),
+                             then the clip's partial sums, one per finalize item */
   int64_t ws_aux;         /* AdaMuon: Newton-Schulz buffers, bf16: M then O [R*C], the iterate
                              X and its successor [m_pad*k_pad] each, A and B [m_pad^2] each;
                              KProdigy: the D statistics' block sums, [2][ceil(pd_ns / KAON_FLAT_ITEM)] */
@@ -385,7 +386,8 @@ int kaon_kprodigy_pass2(const KaonLaunch* L, const KaonHyper* hp, void* stream);
 /* The same steps restricted to the phases whose bit is set in `mask`
  * (bit k = phase k: 1 row statistics, 2 column/row finalize, 3 clip sums,
  * 4 clip divisor, 5 keep-count + momentum absmax, 6 apply; Lion uses 1, 5,
- * 6).  For
+ * 6; Adakaon's and AdaMuon's 3 and 4 are part of the others and launch nothing,
+ * but for the clip of a torch-order step, bit 3).  For
  * profiling one kernel at a time; running all phases in order is the step.
  * No counterpart in the reference, which has no phase boundary to expose. */
 int kaon_adakaon_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask, void* stream);
@@ -395,7 +397,8 @@ int kaon_lion_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask, vo
  * O.  The step is mask 0x37E. */
 int kaon_adamuon_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask, void* stream);
 /* AdaPNM: bits 1-6; phase 3 also records the new positive momentum's int8 row /
- * 4-bit block absmax, phase 5 is the cautious keep count. */
+ * 4-bit block absmax and counts the cautious keeps, phase 5 counts the tensors
+ * whose early count the clip divisor could change (phase 4 marks them). */
 int kaon_adapnm_phases(const KaonLaunch* L, const KaonHyper* hp, uint32_t mask, void* stream);
 
 /* MSAM norm="none" perturbation p += clamp(nan_to_num(factor * dequant(m)), +-bound)

@@ -1,7 +1,8 @@
 // kaon_common.h -- workspace views and device helpers shared by the step
-// kernels' translation units (kaon_step.hip: phases 1-4, the generic phase-5/6
-// kernels, AdaMuon / AdaPNM / KProdigy / MSAM; kaon_fast.hip: the specialized
-// phase-5/6 kernels).  Internal to the library.
+// kernels' translation units (kaon_stats.hip: phase 1; kaon_step.hip: phases 2-4,
+// AdaMuon / AdaPNM / KProdigy / MSAM and the entry points; kaon_fast.hip: the
+// specialized phase-5/6 kernels; kaon_flat.hip: the general ones; kaon_torch.hip:
+// the torch-order sums).  Internal to the library.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -167,9 +168,9 @@ __device__ __forceinline__ void lds_barrier() {
 
 // The tensor's clip divisor max(RMS(U) / clip, 1), RMS(U) = sqrt(ss) / sqrt(n)
 // (_factored.py:84-89 via adakaon.py:1001-1003): formed from the item sums by
-// each workgroup of phases 5 and 6 (Adakaon, AdaMuon; at most a few words, where
-// a launch of its own cost 5 us of a step); AdaPNM's and the torch-order step's
-// clip passes leave it in scalar word 0.
+// each workgroup of phases 5 and 6 (Adakaon, AdaMuon), one sum per KAON_COLITEM
+// columns, where a launch of its own cost 5 us of a step.  AdaPNM's and the
+// torch-order step's clip passes leave it in scalar word 0.
 __device__ __forceinline__ float clip_div(const KaonTensor& T, const Ws& ws, const KaonHyper& hp) {
   const KAON_G float* sc = ws.scal(T);
   if (hp.flags & (KAON_F_PNM | KAON_F_TORCH_ORDER)) return sc[0];

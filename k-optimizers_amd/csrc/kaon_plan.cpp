@@ -276,7 +276,8 @@ extern "C" int kaon_plan(const KaonPlanArgs* args, KaonTensor* descs, int32_t n,
       const int64_t nb = (t.n + t.block4 - 1) / t.block4;
       off = round4(off + 2 * nb);
     }
-    // scalar words: the clip divisor, the keep count, two of KProdigy's / MSAM's,
+    // scalar words: the clip divisor, the keep count, two of KProdigy's / MSAM's /
+    // AdaMuon's / AdaPNM's (KaonTensor.ws_scal),
     // and the clip's algebraic sum: rm, then one partial per finalize item (or one)
     t.ws_scal = off;
     off = round4(off + 5 + (t.factored ? (t.C + KAON_COLITEM - 1) / KAON_COLITEM : 1));
