@@ -142,8 +142,9 @@ def phase_bytes(phase: int, bm: float, wd: bool, opt: str = "adakaon", w: dict |
         if phase in (13, 14):
             return {13: bm, 14: 4.0 + bm}[phase]
     if opt == "adapnm":
-        # both momenta are read by the clip-sum, keep-count and apply passes
-        return {1: 2.0, 3: 2.0 + 2.0 * bm, 5: 2.0 + 2.0 * bm, 6: 6.0 + 3.0 * bm}.get(phase, 0.0)
+        # both momenta are read by the clip-sum pass, which counts the cautious keeps too (the
+        # keep-count pass reads only tensors whose early count does not hold), and by the apply
+        return {1: 2.0, 3: 2.0 + 2.0 * bm, 6: 6.0 + 3.0 * bm}.get(phase, 0.0)
     if phase in (1, 3):
         return 2.0
     if phase == 5:
@@ -221,7 +222,8 @@ def gc_written_elems(opt, name) -> int:
     Lion writes every 2-D+ gradient back; Adakaon (and the Nekaon / MSAM steps over
     it) does so on its native path and, under ``fused=True``, only for the params
     the reference's fused step routes to its native path (``fused_routes_native``).
-    Other optimizers' headline kernels do not store the gradient."""
+    AdaMuon's and AdaPNM's workloads do not store the gradient; KProdigy's apply does,
+    which its workloads' bytes leave out."""
     from kaon_amd.adakaon import fused_routes_native
 
     w = WORKLOADS[name]
@@ -406,7 +408,8 @@ def phase_breakdown(opt, name, reps=5) -> dict[int, float]:
             if key[3] != 2:
                 continue  # the 1-D params' Adakaon plan: a few microseconds
             hp = inner._hyper(group, pdt, gdt)
-            fn, phases = lib.kaon_adamuon_phases, (8, 9, 1, 2, 3, 4, 5, 6)
+            # the clip's sum and divisor are part of phases 1, 2, 5 and 6
+            fn, phases = lib.kaon_adamuon_phases, (8, 9, 1, 2, 5, 6)
         elif WORKLOADS[name]["opt"] == "lion":
             hp = inner._hyper(group, pdt, gdt)
             fn, phases = lib.kaon_lion_phases, (1, 5, 6)
@@ -421,7 +424,8 @@ def phase_breakdown(opt, name, reps=5) -> dict[int, float]:
                 nk = {"remove": True, "bound_old": {gid: float("inf")}, "k": -opt.rho / (opt._mnorm + opt.eps),
                       "climb": False, "eclamp": {}}
             hp = inner._hyper(group, pdt, gdt, nk, gid)
-            fn, phases = lib.kaon_adakaon_phases, (1, 2, 3, 4, 5, 6)
+            # phase 3: the clip of a torch-order step only
+            fn, phases = lib.kaon_adakaon_phases, (1, 2, 3, 5, 6) if hp.flags & _lib.F_TORCH_ORDER else (1, 2, 5, 6)
         s = torch.cuda.current_stream().cuda_stream
         for r in range(reps):
             for ph in phases:
@@ -725,7 +729,7 @@ def main() -> int:
                "config": {"workload": w["desc"], "n_tensors": len(shapes), "n_params": nparam, "params": "f32",
                           "grads": "f32", "momentum": w["kw"]["momentum_dtype"], "parallelism": "none (1 GPU)",
                           "wall_ms_per_step": round(wall / args.steps * 1e3, 4),
-                          "launches_per_step": "5 kernels"}}
+                          "launches_per_step": "4 kernels"}}
         if not args.no_breakdown:
             out["phases_ms"] = {PHASE_NAMES[k]: round(v, 4) for k, v in sorted(phase_breakdown(opt, args.workload)
                                                                                  .items())}

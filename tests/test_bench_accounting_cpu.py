@@ -97,8 +97,11 @@ def test_phase_bytes_per_param():
     # row statistics and clip sums read g once; the finalize and divisor phases touch no per-param data
     assert bench.phase_bytes(1, 1.0, False) == bench.phase_bytes(3, 1.0, False) == 2.0
     assert bench.phase_bytes(2, 1.0, False) == bench.phase_bytes(4, 1.0, False) == 0.0
-    # AdaPNM reads its negative momentum in the clip-sum, keep-count and apply passes
+    # AdaPNM reads its negative momentum in the clip-sum and apply passes; the clip-sum pass
+    # takes the keep count too
     assert bench.phase_bytes(6, 1.0, False, "adapnm") == 9.0
+    assert bench.phase_bytes(3, 1.0, False, "adapnm") == 4.0
+    assert bench.phase_bytes(5, 1.0, False, "adapnm") == 0.0
     # MSAM's norm (m read) and climb (m read, p read + write) passes
     assert bench.phase_bytes(13, 1.0, False, "msam") == 1.0
     assert bench.phase_bytes(14, 1.0, False, "msam") == 5.0
