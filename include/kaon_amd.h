@@ -135,7 +135,8 @@ typedef struct KaonTensor {
   int32_t ngroups;        /* number of runs (column partials) */
   float sqrt_n;           /* (float)sqrt((double)n), the rms divisor (_backend.py:45-47) */
   int32_t vec_rows;       /* 16-byte vector path for row chunks (C % 8 == 0 or one row, aligned) */
-  int32_t vec_flat;       /* 16-byte vector path for flat chunks (all bases aligned) */
+  int32_t vec_flat;       /* all bases 16-byte aligned: the vector path of KProdigy's statistics and
+                             of the MSAM climb (the flat phase-5/6 kernels need no alignment) */
   int32_t ns_tr;          /* AdaMuon: Newton-Schulz iterates on the transpose (R > C) */
   int32_t m_pad, k_pad;   /* AdaMuon: min(R,C) and max(R,C) rounded up to the tile (KAON_NS_TILE,
                              or twice that for big matrices) */
